@@ -1,0 +1,81 @@
+"""The grouped experts of crowded passes at the edges of their tiles: 32 pairs a tile, two tiles a block, 256 weight
+rows a block, whole superblocks of the width. The caller's routing (vitna_cuda_moe_rows_experts takes any) puts 1, 31,
+32, 33, 63, 64, 65, 96, 97 and 129 pairs on the experts of one layer and none on others, for every pair of types, one
+superblock and several, and scales at which the SwiGLU output leaves float16's range on either side.
+
+The oracle: each row's mixture from the checker's norm, projections and SwiGLU on the device's residual rows, to the
+grouped experts' bar of 1e-4 of max |mixture| (float32 sums in another order).
+"""
+import numpy as np
+import pytest
+
+import oracle
+import vitna_amd as va
+from test_gpu_decode import say
+
+pytestmark = pytest.mark.gpu
+
+REL = 1e-4
+COUNTS = [1, 31, 32, 33, 63, 64, 65, 96, 97, 129]
+
+
+def routing(n, E, K, seed):
+    """ids n x K (ascending, distinct): expert i takes COUNTS[i] pairs, the remaining pairs go to the experts after."""
+    rng = np.random.RandomState(seed)
+    left = {e: c for e, c in enumerate(COUNTS)}
+    ids = [[] for _ in range(n)]
+    for e, c in left.items():
+        for r in rng.permutation([r for r in range(n) if len(ids[r]) < K])[:c]:
+            ids[r].append(e)
+    rest = list(range(len(COUNTS), E - 1))  # the last expert takes none
+    for r in range(n):
+        while len(ids[r]) < K:
+            e = rest[rng.randint(len(rest))]
+            if e not in ids[r]:
+                ids[r].append(e)
+    ids = np.sort(np.array(ids, np.int32), axis=1)
+    w = rng.uniform(0.05, 1.0, (n, K)).astype(np.float32)
+    return ids, w
+
+
+def mixture(model, layer, xn, ids, w):
+    experts = model.m.layers[layer].experts
+    out = np.zeros(model.cfg.hidden, np.float32)
+    for e, wt in zip(ids, w):
+        x = experts[int(e)]
+        mv = lambda m, v: oracle.matvec(m.data, m.dtype, v, m.rows, m.cols)
+        out = out + mv(x.down, oracle.silu_mul(mv(x.gate, xn), mv(x.up, xn))) * wt
+    return out
+
+
+@pytest.mark.parametrize("gate_up,down", [(va.Q4_K, va.Q6_K), (va.Q6_K, va.Q4_K), (va.Q4_K, va.Q4_K), (va.Q6_K, va.Q6_K), (va.Q8_0, va.Q8_0)])
+@pytest.mark.parametrize("hidden,inter,k_scale,q8_scale", [(256, 256, 0.01, 0.02 / 127), (512, 768, 3.0, 40.0 / 127), (1024, 256, 2e-4, 5e-3 / 127)])
+def test_tile_edges(gate_up, down, hidden, inter, k_scale, q8_scale):
+    say("tile edges", gate_up, down, hidden, inter, k_scale)
+    n, E, K = 200, 24, 4
+    model = va.Model(va.shape(n_layers=1, hidden=hidden, intermediate=inter, n_heads=4, n_kv_heads=2, head_dim=64, vocab=300, n_experts=E,
+                              n_experts_used=K, renormalize=0, dt_gate_up=gate_up, dt_down=down, norm_std=0.5, k_scale=k_scale,
+                              q8_scale=q8_scale, ctx=n + 8, seqs=1), 977)
+    dev = va.Device(model)
+    try:
+        cfg = model.cfg
+        rows = [((11 * i + 7) % cfg.vocab, i, 0) for i in range(n)]
+        dev.rows_route(rows, 0)
+        norm = np.ctypeslib.as_array(model.m.layers[0].mlp_norm, shape=(hidden,)).copy()
+        x0 = np.stack([dev.residual(i) for i in range(n)])
+        ids, w = routing(n, E, K, 5)
+        dev.rows_experts(0, ids, w)
+        x1 = np.stack([dev.residual(i) for i in range(n)])
+        worst = 0.0
+        for i in range(n):
+            ref = mixture(model, 0, oracle.rmsnorm(x0[i], norm, cfg.rms_eps), ids[i], w[i])
+            want = x0[i].astype(np.float64) + ref
+            r = float(np.max(np.abs(x1[i] - want)) / np.max(np.abs(ref)))
+            # what float32 keeps of a small mixture beside its residual
+            lost = float(np.max(np.abs(want))) * 2.0 ** -23 / float(np.max(np.abs(ref)))
+            worst = max(worst, r)
+            assert r <= REL + lost, ("row", i, r, lost)
+        say("  worst rel err of the mixture", worst)
+    finally:
+        dev.close()
+        model.free()

@@ -11,8 +11,8 @@
  * Two kernels:
  *   skinny_exact_kernel / skinny_wide_kernel (widths a multiple of 256): the
  *     quants enter the MFMA as exact bf16 integers, each scale group keeps its
- *     own MFMA sum and its scale is applied in fp32 (the section "exact-integer
- *     quants" below); the operands come from images in MFMA lane order
+ *     own MFMA sum and its scale is applied in fp32 (skinny_exact.h); the
+ *     operands come from images in MFMA lane order
  *     (skinny_image.h) and the weights from a tiled copy, so every load of a
  *     wave is 1 KB contiguous.
  *   skinny_kernel (other widths): each weight is widened as the reference
@@ -26,20 +26,14 @@
  *     each slice, as the activations' lanes do for token lane % 32.
  * Both stay within 1e-3 of the CPU checker; each projection alone is held to
  * 2e-5 of max |ref| against the widened matrix in float64.
- *
- * The same exact arithmetic serves the grouped experts of crowded passes (64
- * rows and more) on tiles of 32 pairs of one expert (launch_gsx, at the end).
  */
 
 #include "vitna_kernels.h"
 #include "skinny_image.h"
+#include "skinny_exact.h"
 
 #include <algorithm>
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-
-#define SK_TOK 32
 #define SK_NT 2 /* token tiles a block of the exact kernel takes when a pass has many */
 #ifndef SK_NR
 #define SK_NR 2
@@ -282,72 +276,8 @@ __global__ __launch_bounds__(NT == 1 ? 1024 : 256) void skinny_kernel(skinny_arg
     }
 }
 
-/* ---- exact-integer quants ------------------------------------------------ */
-/*
- * Widths a multiple of 256 take this path. A wave owns one tile of 32 weight rows x 32 token rows over one
- * 256-column superblock (one Q4_K or Q6_K block, eight Q8_0 blocks), four units of 64 columns each: the
- * work is a few microseconds of loads a wave, so it is spread as wide as it goes and every load of the
- * wave's weights is issued at once. Within a unit every scale group (Q4_K 32 columns, Q6_K 16, Q8_0 32) keeps its own MFMA sum
- * P over its columns, and the group's scale is applied to P in fp32:
- *   Q8_0  bf16(q) exactly (signed):            acc += d P
- *   Q4_K  bf16(128 + q), q in 0..15:           acc += d sc P  -  (dmin m + 128 d sc) S
- *   Q6_K  bf16(128 + q6), q6 in 0..63:         acc += d sc P  -  160 d sc S
- * where S is the group's sum of the activations. 128 + q is the byte q under the exponent byte of 2^7 (two
- * v_perm_b32 for four weights). The S terms of eight groups go through the matrix cores too, as one
- * 32x32x8 product of the groups' sums (bf16 hi + lo, split on the host side of the pass) by their
- * coefficients, both as three bf16 pieces. S is the sum of the split activations hi + lo, so the offset
- * 128 S cancels exactly what the 128 in the weights added.
- *
- * A unit's k order: lane half kq (lane / 32) of each 16-column MFMA supplies 8 columns, and both operands
- * take them in the same order. Q4_K and Q8_0: the MFMAs of unit u cover columns 64 u + 16 kq + {0, 8} (the
- * first group) and + 32 (the second); Q4_K's byte 32 u + j holds columns 64 u + j (low nibble) and
- * 64 u + 32 + j (high). Q6_K unit u = (h, r0) = (u / 2, u % 2) covers the groups at columns
- * 128 h + 32 r + 16 s, r in {r0, r0 + 2}, s in {0, 1}, of which lane half kq takes columns + 8 kq .. + 8 kq + 7:
- * ql byte 64 h + 32 r0 + 16 s + j holds column 128 h + 32 r0 + 16 s + j (low nibble) and 128 h + 32 (r0 + 2)
- * + 16 s + j (high), qh byte 32 h + 16 s + j its high bits (bits 2 r).
- */
+/* ---- the tiled copy (its layout: skinny_exact.h) ------------------------- */
 
-typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t sx_u2 __attribute__((ext_vector_type(2)));
-
-/* four bytes (each below 128) as bf16 128 + byte */
-__device__ __forceinline__ sx_u2 sx_mag4(uint32_t v) {
-    return sx_u2{__builtin_amdgcn_perm(0x43434343u, v, 0x04010400u), __builtin_amdgcn_perm(0x43434343u, v, 0x04030402u)};
-}
-__device__ __forceinline__ bf16x8 sx_join(sx_u2 a, sx_u2 b) { return __builtin_bit_cast(bf16x8, u32x4{a.x, a.y, b.x, b.y}); }
-/* eight signed bytes as bf16, exactly */
-__device__ __forceinline__ bf16x8 sx_i8(uint32_t a, uint32_t b) {
-    bf16x8 r;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        r[i] = (__bf16)(float)(int8_t)(a >> (8 * i));
-        r[4 + i] = (__bf16)(float)(int8_t)(b >> (8 * i));
-    }
-    return r;
-}
-
-/* One superblock of one 32-row tile: the lane's row's bytes for all four units. */
-template <int DT> struct sx_w;
-template <> struct sx_w<VITNA_DTYPE_Q4_K> { u32x4 q[4], h; };
-template <> struct sx_w<VITNA_DTYPE_Q6_K> { sx_u2 ql[4][2], qh[2][2]; u32x4 sc; uint32_t d; };
-template <> struct sx_w<VITNA_DTYPE_Q8_0> { u32x4 q[4][2], d; };
-
-/* a unit's activations for the lane's token: four 8-column operands, hi and lo, and (when the unit applies
-   S terms) the four group sums of the lane half */
-struct sx_a {
-    u32x4 h[4], l[4];
-    sx_u2 sp[3];
-};
-
-/*
- * The tiled copy: per tile (32 rows; rows past the matrix repeat its last) and superblock, lane l = l32 + 32 kq
- * reads 16-byte pieces at lane-order offsets, so every load is 1 KB contiguous (512 bytes for the per-row
- * fields, which both lane halves read):
- *   Q4_K  [u][lane] q bytes 32 u + 16 kq + 0..15 (u < 4); at 4096 [l32] the 16-byte header
- *   Q6_K  [u][lane] ql bytes 64 (u / 2) + 32 (u % 2) + 16 s + 8 kq + 0..7 for s = 0, 1; at 4096 [h][lane] qh
- *         bytes 32 h + 16 s + 8 kq + 0..7 for s = 0, 1; at 6144 [l32] the 16 scales; at 6656 [l32] d
- *   Q8_0  [2 u + j][lane] q bytes 16 kq + 0..15 of block 8 b + 2 u + j; at 8192 [l32] the 8 blocks' d
- */
 __device__ __forceinline__ uint32_t tile_src(const qmat& m, int tile, int b, int o) {
     /* the byte of the planes that byte o of tile / superblock b copies */
     const int S = m.cols / 256;
@@ -404,186 +334,6 @@ hipError_t launch_tile(const qmat& m, uint8_t* dst, hipStream_t s) {
     if (!tile_bytes(m.dtype) || m.cols % 256 || m.rows < 1) return hipErrorInvalidValue;
     tile_kernel<<<((m.rows + 31) / 32) * (m.cols / 256), 256, 0, s>>>(m, dst);
     return hipGetLastError();
-}
-
-/* The lane's bytes of tile / superblock b from the tiled copy: 1 KB (512-byte) loads in lane order. */
-template <int DT>
-__device__ __forceinline__ void sx_load_w(const qmat& w, int tile, int b, int lane, sx_w<DT>& o) {
-    const uint8_t* T = w.tiled + ((size_t)tile * (w.cols / 256) + b) * (DT == VITNA_DTYPE_Q4_K ? 4608 : DT == VITNA_DTYPE_Q6_K ? 6720 : 8704);
-    const int l32 = lane & 31;
-    if constexpr (DT == VITNA_DTYPE_Q4_K) {
-#pragma unroll
-        for (int u = 0; u < 4; u++) o.q[u] = *reinterpret_cast<const u32x4*>(T + u * 1024 + lane * 16);
-        o.h = *reinterpret_cast<const u32x4*>(T + 4096 + l32 * 16);
-    } else if constexpr (DT == VITNA_DTYPE_Q6_K) {
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const u32x4 v = *reinterpret_cast<const u32x4*>(T + u * 1024 + lane * 16);
-            o.ql[u][0] = sx_u2{v.x, v.y};
-            o.ql[u][1] = sx_u2{v.z, v.w};
-        }
-#pragma unroll
-        for (int h = 0; h < 2; h++) {
-            const u32x4 v = *reinterpret_cast<const u32x4*>(T + 4096 + h * 1024 + lane * 16);
-            o.qh[h][0] = sx_u2{v.x, v.y};
-            o.qh[h][1] = sx_u2{v.z, v.w};
-        }
-        o.sc = *reinterpret_cast<const u32x4*>(T + 6144 + l32 * 16);
-        o.d = *reinterpret_cast<const uint16_t*>(T + 6656 + l32 * 2);
-    } else {
-#pragma unroll
-        for (int v = 0; v < 8; v++) o.q[v >> 1][v & 1] = *reinterpret_cast<const u32x4*>(T + v * 1024 + lane * 16);
-        o.d = *reinterpret_cast<const u32x4*>(T + 8192 + l32 * 16);
-    }
-}
-
-template <int DT> struct sx_unit_sums { static constexpr bool at(int U) { return DT == VITNA_DTYPE_Q4_K ? U == 3 : DT == VITNA_DTYPE_Q6_K ? (U & 1) : false; } };
-
-/* Unit U's operands of token tile tt, superblock b (and the S-term sums when the unit applies them), from the
-   images: every load is 1 KB (512 bytes for the sums) in lane order. */
-template <int DT, int U>
-__device__ __forceinline__ void sx_load_a(const skinny_args& a, int tt, int K, int b, int lane, sx_a& o) {
-    const u32x4* img = reinterpret_cast<const u32x4*>(DT == VITNA_DTYPE_Q6_K ? a.img[1] : a.img[0]) +
-                       ((size_t)tt * (K / 256) + b) * 2048 + (size_t)U * 512 + lane;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        o.h[i] = img[i * 128];
-        o.l[i] = img[i * 128 + 64];
-    }
-    if constexpr (sx_unit_sums<DT>::at(U)) {
-        const sx_u2* sp = DT == VITNA_DTYPE_Q4_K
-                              ? reinterpret_cast<const sx_u2*>(a.s32) + ((size_t)tt * (K / 256) + b) * 192 + lane
-                              : reinterpret_cast<const sx_u2*>(a.s16) + ((size_t)tt * (K / 128) + 2 * b + (U >> 1)) * 192 + lane;
-#pragma unroll
-        for (int i = 0; i < 3; i++) o.sp[i] = sp[64 * i];
-    }
-}
-
-__device__ __forceinline__ void sx_scale(f32x16& acc, float d, const f32x16& P) {
-#pragma unroll
-    for (int r = 0; r < 16; r++) acc[r] = fmaf(d, P[r], acc[r]);
-}
-#define SX_MMA(A, B, C) __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, A), B, C, 0, 0, 0)
-
-/* Q4_K scale and min of group g from the 12 scale bytes (header dwords 1..3) */
-template <int G>
-__device__ __forceinline__ void sx_q4k_sm(const u32x4& h, uint32_t& sc, uint32_t& mn) {
-    if constexpr (G < 4) {
-        sc = (h.y >> (8 * G)) & 63;
-        mn = (h.z >> (8 * G)) & 63;
-    } else {
-        constexpr int j = G - 4;
-        sc = ((h.w >> (8 * j)) & 15) | (((h.y >> (8 * j + 6)) & 3) << 4);
-        mn = ((h.w >> (8 * j + 4)) & 15) | (((h.z >> (8 * j + 6)) & 3) << 4);
-    }
-}
-
-/* the S terms of eight groups: the lane half's four sums times its four coefficients c, each as three bf16
-   pieces, the six products down to 2^-24 of the largest (the offset part of c S cancels against the MFMA sums
-   of 128 + q, so it is carried to fp32 accuracy) */
-__device__ __forceinline__ void sx_sterm(const sx_a& x, const float c[4], f32x16& acc) {
-    s16x4 cp[3];
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const __bf16 p0 = (__bf16)c[i];
-        const float r0 = c[i] - (float)p0;
-        const __bf16 p1 = (__bf16)r0;
-        cp[0][i] = __builtin_bit_cast(short, p0);
-        cp[1][i] = __builtin_bit_cast(short, p1);
-        cp[2][i] = __builtin_bit_cast(short, (__bf16)(r0 - (float)p1));
-    }
-    const s16x4 s0 = __builtin_bit_cast(s16x4, x.sp[0]), s1 = __builtin_bit_cast(s16x4, x.sp[1]), s2 = __builtin_bit_cast(s16x4, x.sp[2]);
-    acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(s2, cp[0], acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(s1, cp[1], acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(s0, cp[2], acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(s1, cp[0], acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(s0, cp[1], acc, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(s0, cp[0], acc, 0, 0, 0);
-}
-
-/* Unit U: its groups' sums and scales into acc; cs carries the superblock's S coefficients (Q4_K) from the
-   units that make them to the unit that applies them. */
-template <int DT, int U>
-__device__ __forceinline__ void sx_compute(const sx_w<DT>& w, const sx_a& x, int kq, f32x16& acc, float cs[8]) {
-    const f32x16 Z = {};
-    if constexpr (DT == VITNA_DTYPE_Q4_K) {
-        constexpr uint32_t M = 0x0f0f0f0fu;
-        const u32x4 q = w.q[U];
-        const bf16x8 a0 = sx_join(sx_mag4(q.x & M), sx_mag4(q.y & M)), a1 = sx_join(sx_mag4(q.z & M), sx_mag4(q.w & M));
-        const bf16x8 b0 = sx_join(sx_mag4((q.x >> 4) & M), sx_mag4((q.y >> 4) & M));
-        const bf16x8 b1 = sx_join(sx_mag4((q.z >> 4) & M), sx_mag4((q.w >> 4) & M));
-        f32x16 P0 = SX_MMA(x.h[0], a0, Z), P1 = SX_MMA(x.h[2], b0, Z);
-        P0 = SX_MMA(x.h[1], a1, P0);
-        P1 = SX_MMA(x.h[3], b1, P1);
-        P0 = SX_MMA(x.l[0], a0, P0);
-        P1 = SX_MMA(x.l[2], b0, P1);
-        P0 = SX_MMA(x.l[1], a1, P0);
-        P1 = SX_MMA(x.l[3], b1, P1);
-        const float d = f16_bits_to_f32(w.h.x & 0xffffu), dmin = f16_bits_to_f32(w.h.x >> 16);
-        uint32_t sc0, mn0, sc1, mn1;
-        sx_q4k_sm<2 * U>(w.h, sc0, mn0);
-        sx_q4k_sm<2 * U + 1>(w.h, sc1, mn1);
-        const float d0 = d * (float)sc0, d1 = d * (float)sc1;
-        sx_scale(acc, d0, P0);
-        sx_scale(acc, d1, P1);
-        cs[2 * U] = -fmaf(128.0f, d0, dmin * (float)mn0);
-        cs[2 * U + 1] = -fmaf(128.0f, d1, dmin * (float)mn1);
-        if constexpr (U == 3) {
-            float c[4];
-#pragma unroll
-            for (int j = 0; j < 4; j++) c[j] = kq ? cs[4 + j] : cs[j];
-            sx_sterm(x, c, acc);
-        }
-    } else if constexpr (DT == VITNA_DTYPE_Q6_K) {
-        constexpr int h = U >> 1, r0 = U & 1;
-        bf16x8 wq[4]; /* groups (r0, 0), (r0, 1), (r0 + 2, 0), (r0 + 2, 1) */
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int s = i & 1, hi = i >> 1, r = r0 + 2 * hi;
-            uint32_t v[2];
-#pragma unroll
-            for (int j = 0; j < 2; j++) {
-                const uint32_t ql = hi ? (w.ql[U][s][j] >> 4) : w.ql[U][s][j];
-                const uint32_t qh = w.qh[h][s][j];
-                const uint32_t top = r == 0 ? qh << 4 : r == 1 ? qh << 2 : r == 2 ? qh : qh >> 2;
-                v[j] = (ql & 0x0f0f0f0fu) | (top & 0x30303030u);
-            }
-            wq[i] = sx_join(sx_mag4(v[0]), sx_mag4(v[1]));
-        }
-        f32x16 P[4];
-#pragma unroll
-        for (int i = 0; i < 4; i++) P[i] = SX_MMA(x.h[i], wq[i], Z);
-#pragma unroll
-        for (int i = 0; i < 4; i++) P[i] = SX_MMA(x.l[i], wq[i], P[i]);
-        const float d = f16_bits_to_f32(w.d);
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const int g = 8 * h + 2 * (r0 + 2 * (i >> 1)) + (i & 1); /* the group's scale index */
-            sx_scale(acc, d * (float)(int8_t)(w.sc[g >> 2] >> (8 * (g & 3))), P[i]);
-        }
-        if constexpr (r0 == 1) {
-            /* the S terms of groups 8 h .. 8 h + 7: lane half kq supplies 8 h + 4 kq .. + 3 */
-            const uint32_t scw = kq ? w.sc[2 * h + 1] : w.sc[2 * h];
-            const float m = -160.0f * d;
-            float c[4];
-#pragma unroll
-            for (int j = 0; j < 4; j++) c[j] = m * (float)(int8_t)(scw >> (8 * j));
-            sx_sterm(x, c, acc);
-        }
-    } else {
-        const bf16x8 a0 = sx_i8(w.q[U][0].x, w.q[U][0].y), a1 = sx_i8(w.q[U][0].z, w.q[U][0].w);
-        const bf16x8 b0 = sx_i8(w.q[U][1].x, w.q[U][1].y), b1 = sx_i8(w.q[U][1].z, w.q[U][1].w);
-        f32x16 P0 = SX_MMA(x.h[0], a0, Z), P1 = SX_MMA(x.h[2], b0, Z);
-        P0 = SX_MMA(x.h[1], a1, P0);
-        P1 = SX_MMA(x.h[3], b1, P1);
-        P0 = SX_MMA(x.l[0], a0, P0);
-        P1 = SX_MMA(x.l[2], b0, P1);
-        P0 = SX_MMA(x.l[1], a1, P0);
-        P1 = SX_MMA(x.l[3], b1, P1);
-        const uint32_t dw = w.d[U];
-        sx_scale(acc, f16_bits_to_f32(dw & 0xffffu), P0);
-        sx_scale(acc, f16_bits_to_f32(dw >> 16), P1);
-    }
 }
 
 /* Superblock b of the lane's weight rows of NR consecutive 32-row tiles (those of them below nr) against NT
@@ -918,23 +668,7 @@ hipError_t launch_skinny(const skinny_args& a, hipStream_t s) {
     return hipGetLastError();
 }
 
-/* ---- grouped experts of crowded passes ------------------------------------ */
-
-/*
- * A pass whose experts hold many pairs each (a prompt's chunk: 1024 rows of top-8 over 128 experts, 64 pairs an
- * expert) runs its experts with the exact arithmetic above on tiles of 32 pairs of one expert, instead of the
- * four-pair tiles of kernels_gmma.hip, so that an expert's weights are read once per 32 pairs rather than once
- * per four. The pairs of each expert (launch_group's lists) are cut into tiles; tile t (of one expert, te[t])
- * is the virtual token tile t of the operand images, which a gather writes from the normalized rows. Gate and up
- * run in one block over the same activations; the block writes the SwiGLU output of its 32 x 32 (pair, row)
- * tile in fp32, whose images the same gather writes for down; down multiplies by the pair's weight into ypart,
- * as kernels_gmma.hip does. The weights come from a copy tiled as the dense matrices' are, experts back to back
- * (expert e's 32-row tile x is tile e I / 32 + x).
- *
- * Reference counterparts: experts_in_rows_kernel model_cuda.cu:2071 and experts_down_rows_kernel
- * model_cuda.cu:2101; the CPU arithmetic checked against is mixture_of_experts engine/src/model.c:745-761 and
- * vitna_silu_mul engine/src/ops.c:283, one row at a time.
- */
+/* ---- the crowded passes' copy of the experts (kernels_tgemm.hip) ------------ */
 
 /* One block a (expert, 32-row tile, superblock): the expert's planes as a matrix of its own. */
 __global__ void gsx_tile_kernel(qmat m, int tiles, uint8_t* __restrict__ dst) {
@@ -955,221 +689,5 @@ hipError_t launch_gsx_tile(const qmat& m, int n_experts, uint8_t* dst, hipStream
     if (!tile_bytes(m.dtype) || m.cols % 256 || m.rows % 32 || n_experts < 1) return hipErrorInvalidValue;
     const int tiles = m.rows / 32;
     gsx_tile_kernel<<<n_experts * tiles * (m.cols / 256), 256, 0, s>>>(m, tiles, dst);
-    return hipGetLastError();
-}
-
-bool gsx_fits(const qmat& gate, const qmat& up, const qmat& down) {
-    auto dt = [](int d) { return d == VITNA_DTYPE_Q8_0 || d == VITNA_DTYPE_Q4_K || d == VITNA_DTYPE_Q6_K; };
-    const int H = gate.cols, I = gate.rows;
-    /* whole superblocks, at most eight a row (one block's waves), whole 32-row tiles */
-    return dt(gate.dtype) && up.dtype == gate.dtype && dt(down.dtype) && up.rows == I && up.cols == H && down.rows == H &&
-           down.cols == I && H % 256 == 0 && I % 256 == 0 && H <= 2048 && I <= 2048;
-}
-
-int gsx_max_tiles(int n, int K, int E) { return (n * K + 31) / 32 + E; }
-
-/* Tile offsets of the experts' pair lists (toff[E + 1]) and the expert of each tile (te[max_tiles], -1 past the
-   last): one block, the first wave scanning the tile counts 64 experts at a time. */
-__global__ __launch_bounds__(256) void gsx_plan_kernel(const int* __restrict__ count, int E, int* __restrict__ toff,
-                                                       int* __restrict__ te, int max_tiles) {
-    __shared__ int off[ROUTE_E_MAX + 1];
-    const int tid = threadIdx.x, lane = tid & 63;
-    if (tid < 64) {
-        int run = 0;
-        for (int e0 = 0; e0 < E; e0 += 64) {
-            const int e = e0 + lane;
-            const int c = e < E ? (count[e] + 31) / 32 : 0;
-            int v = c; /* inclusive scan across the wave */
-#pragma unroll
-            for (int d = 1; d < 64; d <<= 1) {
-                const int o = __shfl_up(v, d, WAVE);
-                if (lane >= d) v += o;
-            }
-            if (e < E) off[e] = run + v - c;
-            run += __shfl(v, 63, WAVE);
-        }
-        if (lane == 0) off[E] = run;
-    }
-    __syncthreads();
-    for (int e = tid; e <= E; e += blockDim.x) toff[e] = off[e];
-    for (int e = tid; e < E; e += blockDim.x)
-        for (int t = off[e]; t < off[e + 1]; t++) te[t] = e;
-    for (int t = off[E] + tid; t < max_tiles; t += blockDim.x) te[t] = -1;
-}
-
-/* The operand images (one column order) and group sums of the virtual token tiles: block (b, t) takes superblock
-   b of tile t. With pairs, token l of tile t is pair toff-relative index 32 (t - toff[e]) + l of expert te[t]
-   (past its count: the last pair again), read from row pair / ROUTE_K_MAX of x; without, it is row 32 t + l of x. */
-__global__ void gsx_image_kernel(const float* __restrict__ x, int K, const int* __restrict__ pairs, const int* __restrict__ count,
-                                 int cap, const int* __restrict__ toff, const int* __restrict__ te, u32x4* __restrict__ imga,
-                                 u32x4* __restrict__ imgb, uint16_t* __restrict__ s32, uint16_t* __restrict__ s16) {
-    const int b = blockIdx.x, t = blockIdx.y;
-    const int e = te[t];
-    if (e < 0) return;
-    const int j0 = 32 * (t - toff[e]), c = count[e];
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        const int item = threadIdx.x + 256 * j, l = item >> 5, c8 = 32 * b + (item & 31);
-        const int row = 32 * t + l;
-        size_t src_row = (size_t)row;
-        if (pairs) src_row = (size_t)(pairs[(size_t)e * cap + min(j0 + l, c - 1)] / ROUTE_K_MAX);
-        const float4* src = reinterpret_cast<const float4*>(x + src_row * K + 8 * c8);
-        const float4 v0 = src[0], v1 = src[1];
-        const float ev[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
-        u32x4 vh, vl;
-        float sum;
-        img_split8(ev, vh, vl, sum);
-        img_put(imga, imgb, row, K, c8, vh, vl);
-        const float t16 = sum + __shfl_xor(sum, 1, WAVE);
-        const float t32 = t16 + __shfl_xor(t16, 2, WAVE);
-        if (!(c8 & 1)) img_sum16(s16, row, K, c8 >> 1, t16);
-        if (!(c8 & 3)) img_sum32(s32, row, K, c8 >> 2, t32);
-    }
-}
-
-/* The KS waves' tiles added in wave order through red ([KS][16][64]); wave wv returns the sums of accumulators
-   wv, wv + KS, ... in out[0], out[1], ... */
-__device__ __forceinline__ void gsx_reduce(const f32x16& acc, float* red, int KS, int wv, int lane, float out[16]) {
-    __syncthreads(); /* red is free */
-#pragma unroll
-    for (int r = 0; r < 16; r++) red[(wv * 16 + r) * 64 + lane] = acc[r];
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < 16; i++) {
-        const int r = wv + i * KS;
-        if (r < 16) {
-            float v = 0.0f;
-            for (int u = 0; u < KS; u++) v += red[(u * 16 + r) * 64 + lane];
-            out[i] = v;
-        }
-    }
-}
-
-/* act[32 t + token][32 x + row] = silu(gate . x) * (up . x) for virtual tile t (expert te[t]) and 32-row tile x
-   (blockIdx.x) of the expert's I rows: KS = H / 256 waves, wave wv on superblock wv of both matrices, each unit's
-   activations loaded once for both. */
-template <int DT>
-__global__ __launch_bounds__(512) void gsx_in_kernel(qmat gate, qmat up, skinny_args sa, const int* __restrict__ te,
-                                                     float* __restrict__ act) {
-    extern __shared__ float red[];
-    const int t = blockIdx.y, e = te[t];
-    if (e < 0) return;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, KS = blockDim.x >> 6, kq = lane >> 5, l32 = lane & 31;
-    const int H = gate.cols, I = gate.rows, x = blockIdx.x, tile = e * (I / 32) + x, b = wv;
-    f32x16 ag = {}, au = {};
-    {
-        sx_w<DT> Wg, Wu;
-        sx_load_w<DT>(gate, tile, b, lane, Wg);
-        sx_load_w<DT>(up, tile, b, lane, Wu);
-        float cg[8], cu[8];
-        sx_a x0, x1;
-        sx_load_a<DT, 0>(sa, t, H, b, lane, x0);
-        sx_load_a<DT, 1>(sa, t, H, b, lane, x1);
-        __builtin_amdgcn_sched_barrier(0);
-        sx_compute<DT, 0>(Wg, x0, kq, ag, cg);
-        sx_compute<DT, 0>(Wu, x0, kq, au, cu);
-        sx_load_a<DT, 2>(sa, t, H, b, lane, x0);
-        __builtin_amdgcn_sched_barrier(0);
-        sx_compute<DT, 1>(Wg, x1, kq, ag, cg);
-        sx_compute<DT, 1>(Wu, x1, kq, au, cu);
-        sx_load_a<DT, 3>(sa, t, H, b, lane, x1);
-        __builtin_amdgcn_sched_barrier(0);
-        sx_compute<DT, 2>(Wg, x0, kq, ag, cg);
-        sx_compute<DT, 2>(Wu, x0, kq, au, cu);
-        sx_compute<DT, 3>(Wg, x1, kq, ag, cg);
-        sx_compute<DT, 3>(Wu, x1, kq, au, cu);
-    }
-    float g[16], u[16];
-    gsx_reduce(ag, red, KS, wv, lane, g);
-    gsx_reduce(au, red, KS, wv, lane, u);
-#pragma unroll
-    for (int i = 0; i < 16; i++) {
-        const int r = wv + i * KS;
-        if (r < 16) {
-            /* accumulator r: token 8 (r / 4) + 4 kq + r % 4 of the tile, row l32 of the tile */
-            const int tok = 8 * (r >> 2) + 4 * kq + (r & 3);
-            const float v = (g[i] / (1.0f + expf(-g[i]))) * u[i];
-            act[(size_t)(32 * t + tok) * I + 32 * x + l32] = v;
-        }
-    }
-}
-
-/* ypart[(row K + slot) H + n] = w_slot (down_e[n] . act[pair]) for the pairs of virtual tile t (past the expert's
-   count: none written) and NR 32-row tiles from NR x of the H rows (each unit's activations loaded once for
-   them): KS = I / 256 waves, wave wv on superblock wv. */
-template <int DT, int NR>
-__global__ __launch_bounds__(512) void gsx_down_kernel(qmat down, skinny_args sa, const int* __restrict__ te,
-                                                       const int* __restrict__ toff, const int* __restrict__ count,
-                                                       const int* __restrict__ pairs, int cap, const route_out* __restrict__ rt,
-                                                       int K, float* __restrict__ ypart) {
-    extern __shared__ float red[];
-    const int t = blockIdx.y, e = te[t];
-    if (e < 0) return;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, KS = blockDim.x >> 6, kq = lane >> 5, l32 = lane & 31;
-    const int H = down.rows, x0 = NR * blockIdx.x;
-    f32x16 acc[NR][1];
-#pragma unroll
-    for (int r = 0; r < NR; r++) acc[r][0] = f32x16{};
-    sx_superblock<DT, 1, NR>(sa, down, e * (H / 32) + x0, NR, t, t + 1, wv, lane, acc);
-    const int j0 = 32 * (t - toff[e]), c = count[e];
-#pragma unroll
-    for (int wr = 0; wr < NR; wr++) {
-        float v[16];
-        gsx_reduce(acc[wr][0], red, KS, wv, lane, v);
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int r = wv + i * KS;
-            if (r < 16) {
-                const int j = j0 + 8 * (r >> 2) + 4 * kq + (r & 3);
-                if (j < c) {
-                    const int p = pairs[(size_t)e * cap + j], row = p / ROUTE_K_MAX, slot = p % ROUTE_K_MAX;
-                    ypart[((size_t)row * K + slot) * H + 32 * (x0 + wr) + l32] = rt[row].weights[slot] * v[i];
-                }
-            }
-        }
-    }
-}
-
-hipError_t launch_gsx(const gsx_args& a, hipStream_t s) {
-    if (!gsx_fits(a.gate, a.up, a.down) || !a.gate.tiled || !a.up.tiled || !a.down.tiled || a.K < 1 || a.K > ROUTE_K_MAX ||
-        a.E < 1 || a.E > ROUTE_E_MAX || a.n < 1 || a.cap < a.n || a.max_tiles < gsx_max_tiles(a.n, a.K, a.E))
-        return hipErrorInvalidValue;
-    const int H = a.gate.cols, I = a.gate.rows, T = gsx_max_tiles(a.n, a.K, a.E);
-    gsx_plan_kernel<<<1, 256, 0, s>>>(a.count, a.E, a.toff, a.te, T);
-    const bool in_b = a.gate.dtype == VITNA_DTYPE_Q6_K, dn_b = a.down.dtype == VITNA_DTYPE_Q6_K;
-    u32x4* ii = reinterpret_cast<u32x4*>(a.img_in);
-    u32x4* ia = reinterpret_cast<u32x4*>(a.img_act);
-    gsx_image_kernel<<<dim3(H / 256, T), 256, 0, s>>>(a.xn, H, a.pairs, a.count, a.cap, a.toff, a.te, in_b ? nullptr : ii,
-                                                      in_b ? ii : nullptr, a.s32, a.s16);
-    skinny_args si{};
-    si.img[0] = si.img[1] = a.img_in;
-    si.s32 = reinterpret_cast<const uint32_t*>(a.s32);
-    si.s16 = reinterpret_cast<const uint32_t*>(a.s16);
-    const int ksi = H / 256, ksd = I / 256;
-    const dim3 gi(I / 32, T), gd(H / 32, T);
-    switch (a.gate.dtype) {
-    case VITNA_DTYPE_Q4_K: gsx_in_kernel<VITNA_DTYPE_Q4_K><<<gi, 64 * ksi, ksi * 4096, s>>>(a.gate, a.up, si, a.te, a.act); break;
-    case VITNA_DTYPE_Q6_K: gsx_in_kernel<VITNA_DTYPE_Q6_K><<<gi, 64 * ksi, ksi * 4096, s>>>(a.gate, a.up, si, a.te, a.act); break;
-    default: gsx_in_kernel<VITNA_DTYPE_Q8_0><<<gi, 64 * ksi, ksi * 4096, s>>>(a.gate, a.up, si, a.te, a.act); break;
-    }
-    gsx_image_kernel<<<dim3(I / 256, T), 256, 0, s>>>(a.act, I, nullptr, a.count, a.cap, a.toff, a.te, dn_b ? nullptr : ia,
-                                                      dn_b ? ia : nullptr, a.s32, a.s16);
-    skinny_args sd{};
-    sd.img[0] = sd.img[1] = a.img_act;
-    sd.s32 = reinterpret_cast<const uint32_t*>(a.s32);
-    sd.s16 = reinterpret_cast<const uint32_t*>(a.s16);
-    /* two 32-row tiles a block for K-quant down weights (Q8_0's two do not fit the registers) */
-    const dim3 gd2(H / 64, T);
-    switch (a.down.dtype) {
-    case VITNA_DTYPE_Q4_K:
-        gsx_down_kernel<VITNA_DTYPE_Q4_K, 2><<<gd2, 64 * ksd, ksd * 4096, s>>>(a.down, sd, a.te, a.toff, a.count, a.pairs, a.cap, a.rt, a.K, a.ypart);
-        break;
-    case VITNA_DTYPE_Q6_K:
-        gsx_down_kernel<VITNA_DTYPE_Q6_K, 2><<<gd2, 64 * ksd, ksd * 4096, s>>>(a.down, sd, a.te, a.toff, a.count, a.pairs, a.cap, a.rt, a.K, a.ypart);
-        break;
-    default:
-        gsx_down_kernel<VITNA_DTYPE_Q8_0, 1><<<gd, 64 * ksd, ksd * 4096, s>>>(a.down, sd, a.te, a.toff, a.count, a.pairs, a.cap, a.rt, a.K, a.ypart);
-        break;
-    }
     return hipGetLastError();
 }
