@@ -79,3 +79,53 @@ def test_tile_edges(gate_up, down, hidden, inter, k_scale, q8_scale):
     finally:
         dev.close()
         model.free()
+
+
+def fast_bound(model, layer, xn, ids, w):
+    """A fast pass's mixture and its bound: activations, weights and SwiGLU outputs each within 2^-11 of themselves (f16), so
+    a product within 2^-10; the gate's and up's error carried through SwiGLU to first order, and 5 % for the rest."""
+    e10 = 2.0 ** -10
+    out, bound = np.zeros(model.cfg.hidden), np.zeros(model.cfg.hidden)
+    for e, wt in zip(ids, w):
+        x = model.m.layers[layer].experts[int(e)]
+        G, U, D = (oracle.widen(m.bytes(), m.dtype, m.rows * m.cols).reshape(m.rows, m.cols).astype(np.float64) for m in (x.gate, x.up, x.down))
+        xd = xn.astype(np.float64)
+        g, u = G @ xd, U @ xd
+        dg, du = e10 * (np.abs(G) @ np.abs(xd)), e10 * (np.abs(U) @ np.abs(xd))
+        sg = 1.0 / (1.0 + np.exp(-np.clip(g, -700, 700)))
+        a = g * sg * u
+        # |silu'| is at most 1.1 everywhere
+        da = 1.1 * np.abs(u) * dg + (np.abs(g * sg) + 1.1 * dg) * du
+        out += wt * (D @ a)
+        bound += abs(wt) * (np.abs(D) @ (da + e10 * np.abs(a)))
+    return out, 1.05 * bound
+
+
+@pytest.mark.parametrize("gate_up,down", [(va.Q4_K, va.Q6_K), (va.Q6_K, va.Q4_K)])
+@pytest.mark.parametrize("hidden,inter", [(256, 256), (512, 768)])
+def test_fast_tile_edges(gate_up, down, hidden, inter):
+    """The same pairs an expert through a --precision fast model: blocks of four tiles of one expert."""
+    say("fast tile edges", gate_up, down, hidden, inter)
+    n, E, K = 200, 24, 4
+    model = va.Model(va.shape(n_layers=1, hidden=hidden, intermediate=inter, n_heads=4, n_kv_heads=2, head_dim=64, vocab=300, n_experts=E,
+                              n_experts_used=K, renormalize=0, dt_gate_up=gate_up, dt_down=down, norm_std=0.5, ctx=n + 8, seqs=1), 978)
+    dev = va.Device(model, fast=True)
+    try:
+        cfg = model.cfg
+        rows = [((11 * i + 7) % cfg.vocab, i, 0) for i in range(n)]
+        dev.rows_route(rows, 0)
+        norm = np.ctypeslib.as_array(model.m.layers[0].mlp_norm, shape=(hidden,)).copy()
+        x0 = np.stack([dev.residual(i) for i in range(n)])
+        ids, w = routing(n, E, K, 6)
+        dev.rows_experts(0, ids, w)
+        worst = 0.0
+        for i in range(0, n, 3):
+            ref, bound = fast_bound(model, 0, oracle.rmsnorm(x0[i], norm, cfg.rms_eps), ids[i], w[i])
+            got = dev.residual(i).astype(np.float64) - x0[i]
+            r = float(np.max(np.abs(got - ref) / bound))
+            worst = max(worst, r)
+            assert r <= 1.0, ("row", i, r)
+        say("  worst share of the bound", worst)
+    finally:
+        dev.close()
+        model.free()

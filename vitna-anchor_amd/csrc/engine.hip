@@ -2147,6 +2147,21 @@ static hipError_t enqueue_rows_attention(vitna_cuda_model* g, int layer, int n, 
    to the exact kernels' but not their bits. */
 static bool rows_fast(const vitna_cuda_model* g, int n) { return g->fast && (size_t)n >= g->fast_rows; }
 
+/* Whether a pass of n rows runs layer's experts on the tiles of kernels_tgemm.hip. A fast pass does for K-quant experts;
+   Q8_0's keep the prefill's kernel, which widens each wave's own weights. */
+static bool rows_tiled(const vitna_cuda_model* g, int layer, int n) {
+    const dlayer& d = g->L[layer];
+    if (n < GSX_ROWS || !d.sx_gate) return false;
+    return !rows_fast(g, n) || (d.gate.dtype != VITNA_DTYPE_Q8_0 && d.down.dtype != VITNA_DTYPE_Q8_0);
+}
+
+/* A fast pass's working buffers for the layers that take the prefill's kernels, if any does. */
+static bool fast_reserve(vitna_cuda_model* g, size_t n, char* err, size_t err_len) {
+    for (int l = 0; l < g->NL; l++)
+        if (!rows_tiled(g, l, (int)n)) return prefill_reserve(g, n, err, err_len);
+    return true;
+}
+
 /* The experts of a fast pass of n rows as rt[0..n) routes them: the normalized rows (g->xn) rounded to bf16, the
    (row, slot) pairs grouped by expert, the prefill's grouped GEMM (gate/up with SwiGLU, then down times the
    weight), each row's K parts added onto its residual row in slot order. The working buffers are the prefill's,
@@ -2178,14 +2193,14 @@ static hipError_t enqueue_rows_experts(vitna_cuda_model* g, int layer, int n, bo
     if (!rt) rt = g->rt;
     hipError_t e = launch_group(rt, n, g->E, g->K, ROWS_MAX, g->grp_count, g->grp_pairs, g->stream);
     if (e != hipSuccess) return e;
-    if (n >= GSX_ROWS && d.sx_gate) {
+    if (rows_tiled(g, layer, n)) {
         /* a crowded pass: tiles of 32 pairs of one expert */
         gsx_args x{};
         x.gate = d.gate; x.gate.tiled = d.sx_gate;
         x.up = d.up; x.up.tiled = d.sx_up;
         x.down = d.down; x.down.tiled = d.sx_down;
         x.xn = g->xn; x.rt = rt; x.count = g->grp_count; x.pairs = g->grp_pairs;
-        x.E = g->E; x.K = g->K; x.cap = ROWS_MAX; x.n = n;
+        x.E = g->E; x.K = g->K; x.cap = ROWS_MAX; x.n = n; x.fast = rows_fast(g, n);
         x.toff = g->gsx_toff; x.te = g->gsx_te; x.tb = g->gsx_tb; x.max_tiles = gsx_max_tiles(ROWS_MAX, g->K, g->E);
         x.img_in = g->gsx_img_in; x.img_act = g->gsx_img_act; x.sums = g->gsx_sums; x.xscale = d.mlp_scale; x.inv = g->gsx_inv;
         x.act = g->gsx_act; x.ypart = g->ypart;
@@ -2552,8 +2567,9 @@ extern "C" bool vitna_cuda_moe_rows_experts(struct vitna_cuda_model* g, size_t l
         return put_routing(g, n, ids, weights, k, err, err_len) &&
                check_launch(g, enqueue_exact_experts(g, (int)layer, (int)n), "the rows' experts", err, err_len);
     if (rows_fast(g, (int)n)) {
-        if (!prefill_reserve(g, n, err, err_len) || !put_routing(g, n, ids, weights, k, err, err_len)) return false;
-        return check_launch(g, enqueue_fast_experts(g, (int)layer, (int)n, g->rt), "the rows' experts (grouped GEMM)", err, err_len);
+        if (!fast_reserve(g, n, err, err_len) || !put_routing(g, n, ids, weights, k, err, err_len)) return false;
+        return check_launch(g, rows_tiled(g, (int)layer, (int)n) ? enqueue_rows_experts(g, (int)layer, (int)n, false)
+                                                                 : enqueue_fast_experts(g, (int)layer, (int)n, g->rt), "the rows' experts (grouped GEMM)", err, err_len);
     }
     if (!put_routing(g, n, ids, weights, k, err, err_len)) return false;
     return check_launch(g, enqueue_rows_experts(g, (int)layer, (int)n, false), "the rows' experts", err, err_len);
@@ -2591,8 +2607,9 @@ static hipError_t enqueue_rows_step_body(vitna_cuda_model* g, int n, int head) {
         if (fast) {
             if (e == hipSuccess) e = enqueue_route(g, l, g->rlogits, n, g->x, g->xn, true, nullptr, rt);
             if (e == hipSuccess && n == 1) e = launch_topk(g->rlogits, 1, g->E, g->K, g->renorm, rt, g->stream);
-            if (e == hipSuccess) e = enqueue_fast_experts(g, l, n, rt);
-            pending = nullptr;
+            const bool tiled = rows_tiled(g, l, n);
+            if (e == hipSuccess) e = tiled ? enqueue_rows_experts(g, l, n, true, true, rt) : enqueue_fast_experts(g, l, n, rt);
+            pending = tiled ? g->ypart : nullptr;
             continue;
         }
         /* several rows: the top-k kernel also splits the normed rows for the grouped experts */
@@ -2610,7 +2627,7 @@ static hipError_t enqueue_rows_step_body(vitna_cuda_model* g, int n, int head) {
 static bool ensure_rows_graph(vitna_cuda_model* g, int n, int head, char* err, size_t err_len) {
     if (!ensure_tiled(g, err, err_len)) return false;
     /* a fast pass's working buffers exist before the capture (growing them later would free what the graph uses) */
-    if (rows_fast(g, n) && !prefill_reserve(g, (size_t)n, err, err_len)) return false;
+    if (rows_fast(g, n) && !fast_reserve(g, (size_t)n, err, err_len)) return false;
     const bool fast = rows_fast(g, n);
     int pick = 0;
     for (int i = 0; i < ROWS_GRAPHS; i++) {

@@ -28,6 +28,13 @@
  * first loads most of its life. One layer's experts of a 1024-row pass (top-8
  * of 128, 2048 x 768; kernel trace): gate/up in Q4_K 293 -> 163 us, down in
  * Q6_K 243 -> 173 us; 333 rows in Q8_0 155 -> 112 and 113 -> 74 us.
+ *
+ * A --precision fast pass takes the activations' hi alone: a wave's second
+ * token tile takes the place of the first one's lo, so a block holds four
+ * tiles of one expert and each weight is unpacked for two. Against the bf16
+ * GEMM that widened each K-quant weight in float32 (kernels_prefill.hip): 246
+ * -> 131 and 181 -> 135 us at the same sizes, the error against 64 bits of a
+ * two-layer pass 6e-3 -> 4e-4 (f16 keeps 11 bits, bf16 8).
  */
 
 #include "vitna_kernels.h"
@@ -52,8 +59,8 @@ template <int DT> struct tg_lds;
 template <> struct tg_lds<VITNA_DTYPE_Q4_K> {
     static constexpr int TB = 4608, WU = 1024, HDR_LANES = 32;
     static constexpr int HDR = 4 * (TG_T * 8192 + TG_R * WU); /* [8][512] */
-    static constexpr int SUMS = HDR + TG_R * 512;             /* [2][1024] */
-    static constexpr int BYTES = SUMS + TG_T * 1024;
+    static constexpr int SUMS = HDR + TG_R * 512;             /* [2][1024], FAST [4][1024] */
+    static constexpr int BYTES = SUMS + 2 * TG_T * 1024;
     static constexpr int loads(int u) { return TG_T + 1 + (u == 0); }
 };
 template <> struct tg_lds<VITNA_DTYPE_Q6_K> {
@@ -95,12 +102,12 @@ __device__ __forceinline__ void tg_wait() {
 
 /* Part PART of unit U of superblock b into its slot: 0 and 1 the token tiles' images, 2 the weights and what the
    superblock has once. */
-template <int DT, int U, int PART>
+template <int DT, bool FAST, int U, int PART>
 __device__ __forceinline__ void tg_part(const tg_src& s, int b, uint32_t lds, int wv, int lane) {
     typedef tg_lds<DT> L;
     const uint32_t off = 16 * lane, slot = lds + U * (TG_T * 8192 + TG_R * L::WU);
     if constexpr (PART < TG_T) {
-        tg_dma(s.img[PART] + (size_t)b * 32768 + U * 8192, off, slot + PART * 8192 + wv * 1024);
+        tg_dma(s.img[PART] + (size_t)b * (FAST ? 16384 : 32768) + U * (FAST ? 4096 : 8192), off, slot + PART * 8192 + wv * 1024);
     } else {
         const uint8_t* w = s.wt + (size_t)b * L::TB;
 #pragma unroll
@@ -109,19 +116,19 @@ __device__ __forceinline__ void tg_part(const tg_src& s, int b, uint32_t lds, in
             tg_dma(w + 4096 + (U / 2) * 1024, off, lds + L::QH + ((U / 2) * TG_R + wv) * 1024);
         if constexpr (U == 0) {
             if (lane < L::HDR_LANES) tg_dma(w + 4 * L::WU + (DT == VITNA_DTYPE_Q6_K ? 2048 : 0), off, lds + L::HDR + wv * L::HDR_LANES * 16);
-            if (DT == VITNA_DTYPE_Q4_K && wv < TG_T) tg_dma(s.sums + (size_t)b * 1024, off, lds + L::SUMS + wv * 1024);
+            if (DT == VITNA_DTYPE_Q4_K && wv < (FAST ? 2 : 1) * TG_T) tg_dma(s.sums + (size_t)b * 1024, off, lds + L::SUMS + wv * 1024);
         }
     }
 }
-template <int DT, int U>
+template <int DT, bool FAST, int U>
 __device__ __forceinline__ void tg_issue(const tg_src& s, int b, uint32_t lds, int wv, int lane) {
-    tg_part<DT, U, 0>(s, b, lds, wv, lane);
-    tg_part<DT, U, 1>(s, b, lds, wv, lane);
-    tg_part<DT, U, 2>(s, b, lds, wv, lane);
+    tg_part<DT, FAST, U, 0>(s, b, lds, wv, lane);
+    tg_part<DT, FAST, U, 1>(s, b, lds, wv, lane);
+    tg_part<DT, FAST, U, 2>(s, b, lds, wv, lane);
 }
 
 /* The lane's operands of unit U from its slot: half N of the activations of token tile tg (hi and lo of its two
-   steps), the weight tile at LDS index r. */
+   steps; FAST: hi of its two tiles), the weight tile at LDS index r. */
 struct tg_a {
     u32x4 h[2], l[2];
 };
@@ -173,12 +180,15 @@ __device__ __forceinline__ void tg_keep(T& v) { asm volatile("" : "+v"(v)); }
    that is not live (its token tile lies past the rows) loads its share and computes nothing.
    A wave issues in order, so a step (half a unit) keeps its three parts apart and interleaves them: the products
    of this step on operands made before, the unpacking of the next step's weights, and the scaling of the last
-   finished products; and it reads from LDS what the next step multiplies and the one after it unpacks. */
-template <int DT>
+   finished products; and it reads from LDS what the next step multiplies and the one after it unpacks.
+   FAST: activations in f16 alone (hi). A wave then takes two token tiles, the second's hi in the place of the first's
+   lo, against weights that are unpacked once for both, and what Q6_K's rounding leaves is dropped. */
+template <int DT, bool FAST>
 __device__ __forceinline__ void tg_body(const tg_src& s, int S, const uint8_t* lds, uint32_t base, int wv, int lane, int r0, int tg, bool live,
-                                        f32x16 (&acc)[2]) {
+                                        f32x16 (&acc)[FAST ? 2 : 1][2]) {
     typedef tg_lds<DT> L;
-    constexpr bool Q4 = DT == VITNA_DTYPE_Q4_K, Q6 = DT == VITNA_DTYPE_Q6_K, Q8 = DT == VITNA_DTYPE_Q8_0;
+    constexpr bool Q4 = DT == VITNA_DTYPE_Q4_K, Q6 = DT == VITNA_DTYPE_Q6_K && !FAST, Q8 = DT == VITNA_DTYPE_Q8_0;
+    constexpr int NT = FAST ? 2 : 1;
     auto top = [&](auto u, int b) {
         constexpr int U = decltype(u)::value;
         /* the next unit has landed, the loads of the one after it may still run; the unit loaded from here on goes to
@@ -188,16 +198,16 @@ __device__ __forceinline__ void tg_body(const tg_src& s, int S, const uint8_t* l
     };
     auto load = [&](auto u, auto part, int b) {
         constexpr int U = decltype(u)::value, PART = decltype(part)::value;
-        if constexpr (U == 0) tg_part<DT, 3, PART>(s, b, base, wv, lane);
-        else if (b + 1 < S) tg_part<DT, (U + 3) & 3, PART>(s, b + 1, base, wv, lane);
+        if constexpr (U == 0) tg_part<DT, FAST, 3, PART>(s, b, base, wv, lane);
+        else if (b + 1 < S) tg_part<DT, FAST, (U + 3) & 3, PART>(s, b + 1, base, wv, lane);
     };
     std::integral_constant<int, 0> u0;
     std::integral_constant<int, 1> u1;
     std::integral_constant<int, 2> u2;
     std::integral_constant<int, 3> u3;
-    tg_issue<DT, 0>(s, 0, base, wv, lane);
-    tg_issue<DT, 1>(s, 0, base, wv, lane);
-    tg_issue<DT, 2>(s, 0, base, wv, lane);
+    tg_issue<DT, FAST, 0>(s, 0, base, wv, lane);
+    tg_issue<DT, FAST, 1>(s, 0, base, wv, lane);
+    tg_issue<DT, FAST, 2>(s, 0, base, wv, lane);
     tg_wait<L::loads(1) + L::loads(2)>();
     if (!live) {
         auto unit = [&](auto u, int b) {
@@ -218,12 +228,13 @@ __device__ __forceinline__ void tg_body(const tg_src& s, int S, const uint8_t* l
     tg_a x[2];       /* the activations of this step and the next, by the step's parity */
     th_b<DT> o[2];   /* the weights of this step */
     h8 mins[2];      /* Q4_K: a superblock's minimums */
-    u32x4 sums;      /* and its sums */
-    f32x16 P[2] = {}, M[2]; /* the products, with their scale dP once they are finished, and Q4_K's of the minimums */
+    u32x4 sums[NT];  /* and its sums */
+    f32x16 P[NT][2] = {}, M[2]; /* the products, with their scale dP once they are finished, and Q4_K's of the minimums */
     float dP[2] = {0.0f, 0.0f}, dM[2] = {0.0f, 0.0f};
     auto start = [&](const sx_w<DT>(&ws)[2]) { /* a superblock's minimums and sums */
         if constexpr (Q4) {
-            sums = *(reinterpret_cast<const u32x4*>(lds + L::SUMS + tg * 1024) + lane);
+#pragma unroll
+            for (int t = 0; t < NT; t++) sums[t] = *(reinterpret_cast<const u32x4*>(lds + L::SUMS + (NT * tg + t) * 1024) + lane);
             mins[0] = th_mins(th_header(ws[0]));
             mins[1] = th_mins(th_header(ws[1]));
         }
@@ -241,7 +252,9 @@ __device__ __forceinline__ void tg_body(const tg_src& s, int S, const uint8_t* l
     for (int b = 0; b < S; b++) {
         auto step = [&](auto u, auto half) {
             constexpr int U = decltype(u)::value, N = decltype(half)::value, V = (U + 1) & 3;
-            constexpr bool first = U == 0 && N == 0, mid = U == 0 && N == 1, last = U == 3 && N == 1;
+            constexpr bool first = U == 0 && N == 0, last = U == 3 && N == 1;
+            /* a token tile's products of the minimums in one of the first steps, their scale in the next */
+            constexpr int mt = Q4 && 2 * U + N < NT ? 2 * U + N : -1, ms = Q4 && 2 * U + N >= 1 && 2 * U + N <= NT ? 2 * U + N - 1 : -1;
             __builtin_amdgcn_sched_barrier(0);
             sx_w<DT>(&ws)[2] = U == 3 ? wn : w; /* the next unit's */
             if constexpr (N == 0) {
@@ -252,42 +265,45 @@ __device__ __forceinline__ void tg_body(const tg_src& s, int S, const uint8_t* l
             tg_read_w<DT, V, N>(lds, r0, lane, ws[0]);
             tg_read_w<DT, V, N>(lds, r0 + 1, lane, ws[1]);
             const tg_a xs = x[N];
-            if constexpr (Q4 && first) {
-#pragma unroll
-                for (int i = 0; i < 2; i++) {
-                    M[i] = TH_MMA(sums, mins[i], f32x16{});
-                    dM[i] = th_dmin(w[i]);
-                }
-            }
             /* the finished products' scale */
             if constexpr (Q8 || first) {
 #pragma unroll
-                for (int i = 0; i < 2; i++) {
-                    sx_scale(acc[i], dP[i], P[i]);
-                    tg_keep(acc[i]);
-                    P[i] = f32x16{};
-                }
-            } else if constexpr (Q4 && mid) {
+                for (int t = 0; t < NT; t++)
+#pragma unroll
+                    for (int i = 0; i < 2; i++) {
+                        sx_scale(acc[t][i], dP[i], P[t][i]);
+                        tg_keep(acc[t][i]);
+                        P[t][i] = f32x16{};
+                    }
+            }
+            if constexpr (ms >= 0) {
 #pragma unroll
                 for (int i = 0; i < 2; i++) {
-                    sx_scale(acc[i], dM[i], M[i]);
-                    tg_keep(acc[i]);
+                    sx_scale(acc[ms][i], dM[i], M[i]);
+                    tg_keep(acc[ms][i]);
+                }
+            }
+            if constexpr (mt >= 0) {
+#pragma unroll
+                for (int i = 0; i < 2; i++) {
+                    M[i] = TH_MMA(sums[mt], mins[i], f32x16{});
+                    if (mt == 0) dM[i] = th_dmin(w[i]);
                 }
             }
             /* this step's products */
 #pragma unroll
             for (int k = 0; k < 2; k++)
 #pragma unroll
-                for (int i = 0; i < 2; i++) P[i] = TH_MMA(xs.h[k], o[i].o[k], P[i]);
+                for (int i = 0; i < 2; i++) P[0][i] = TH_MMA(xs.h[k], o[i].o[k], P[0][i]);
 #pragma unroll
             for (int k = 0; k < 2; k++)
 #pragma unroll
-                for (int i = 0; i < 2; i++) P[i] = TH_MMA(xs.l[k], o[i].o[k], P[i]);
+                for (int i = 0; i < 2; i++) P[NT - 1][i] = TH_MMA(xs.l[k], o[i].o[k], P[NT - 1][i]);
             if constexpr (Q6) {
 #pragma unroll
                 for (int k = 0; k < 2; k++)
 #pragma unroll
-                    for (int i = 0; i < 2; i++) P[i] = TH_MMA(xs.h[k], o[i].r[k], P[i]);
+                    for (int i = 0; i < 2; i++) P[0][i] = TH_MMA(xs.h[k], o[i].r[k], P[0][i]);
             }
             /* the next step's weights (past the last superblock, whatever the slots hold: not used) */
             th_b<DT> on[2];
@@ -334,24 +350,27 @@ __device__ __forceinline__ void tg_body(const tg_src& s, int S, const uint8_t* l
         w[0] = wn[0];
         w[1] = wn[1];
     }
-    sx_scale(acc[0], dP[0], P[0]);
-    sx_scale(acc[1], dP[1], P[1]);
+#pragma unroll
+    for (int t = 0; t < NT; t++)
+#pragma unroll
+        for (int i = 0; i < 2; i++) sx_scale(acc[t][i], dP[i], P[t][i]);
 }
 
 /* What the kernels read: the rows' operand images (img, tile_half.h's values in skinny_image.h's layout, order B for
-   Q6_K) and, for Q4_K, group sums ([tile][superblock][64][8] f16). */
+   Q6_K; FAST: the hi pieces alone) and, for Q4_K, group sums ([tile][superblock][64][8] f16). */
 struct tg_images {
     const uint8_t *img, *sums;
 };
 
-/* One wave's sources: token tiles tt of S0 superblocks each, its weight tile, from superblock b0 on. */
-template <int DT>
-__device__ __forceinline__ tg_src tg_sources(const tg_images& a, const int (&tt)[TG_T], const uint8_t* tile, int S0, int b0, int wv) {
+/* One wave's sources: token tiles tt (two, FAST four) of S superblocks each, its weight tile. */
+template <int DT, bool FAST>
+__device__ __forceinline__ tg_src tg_sources(const tg_images& a, const int (&tt)[2 * TG_T], const uint8_t* tile, int S, int wv) {
     tg_src s;
 #pragma unroll
-    for (int j = 0; j < TG_T; j++) s.img[j] = a.img + ((size_t)tt[j] * S0 + b0) * 32768 + wv * 1024;
-    s.wt = tile + (size_t)b0 * tg_lds<DT>::TB;
-    s.sums = a.sums + ((size_t)tt[wv & 1] * S0 + b0) * 1024;
+    for (int j = 0; j < TG_T; j++)
+        s.img[j] = FAST ? a.img + (size_t)tt[2 * j + (wv & 1)] * S * 16384 + (wv >> 1) * 1024 : a.img + (size_t)tt[j] * S * 32768 + wv * 1024;
+    s.wt = tile;
+    s.sums = a.sums + (size_t)tt[wv & (FAST ? 3 : 1)] * S * 1024;
     return s;
 }
 
@@ -373,7 +392,7 @@ __device__ __forceinline__ int tg_item(int n) {
  * expert) runs its experts on tiles of 32 pairs of one expert, instead of the four-pair tiles of kernels_gmma.hip,
  * with the f16 arithmetic of tile_half.h. The pairs of each expert (launch_group's lists) are cut into tiles; tile t
  * (of one expert, te[t]) is the virtual token tile t of the operand images, which a gather writes from the
- * normalized rows. A token block is up to two tiles of one expert. Gate and up run in one block over the same
+ * normalized rows. A token block is up to two tiles of one expert (a fast pass: four). Gate and up run in one block over the same
  * activations; the block writes the SwiGLU output in fp32, whose images gsx_act_image_kernel writes for down; down
  * multiplies by the pair's weight into ypart, as kernels_gmma.hip does. The weights come from a copy tiled as the
  * dense matrices' are, experts back to back (expert e's 32-row tile x is tile e I / 32 + x).
@@ -391,14 +410,15 @@ int gsx_max_tiles(int n, int K, int E) { return (n * K + 31) / 32 + E; }
 int gsx_max_blocks(int n, int K, int E) { return (n * K + 63) / 64 + E; }
 
 /* Tile offsets of the experts' pair lists (toff[E + 1]), the expert of each tile (te[max_tiles], -1 past the
-   last) and the first tile of each token block (tb, their number at n_tb): one block, the first wave scanning the
+   last) and the first tile of each token block of up to `block` tiles (tb, their number at n_tb): one block, the first wave scanning the
    tile counts, the second the block counts, 64 experts at a time. */
 __global__ __launch_bounds__(256) void gsx_plan_kernel(const int* __restrict__ count, int E, int* __restrict__ toff,
-                                                       int* __restrict__ te, int max_tiles, int* __restrict__ tb, int* __restrict__ n_tb) {
+                                                       int* __restrict__ te, int max_tiles, int block, int* __restrict__ tb,
+                                                       int* __restrict__ n_tb) {
     __shared__ int off[2][ROUTE_E_MAX + 1];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     if (wv < 2) {
-        const int per = wv ? 64 : 32;
+        const int per = wv ? 32 * block : 32;
         int run = 0;
         for (int e0 = 0; e0 < E; e0 += 64) {
             const int e = e0 + lane;
@@ -418,45 +438,60 @@ __global__ __launch_bounds__(256) void gsx_plan_kernel(const int* __restrict__ c
     for (int e = tid; e <= E; e += blockDim.x) toff[e] = off[0][e];
     for (int e = tid; e < E; e += blockDim.x) {
         for (int t = off[0][e]; t < off[0][e + 1]; t++) te[t] = e;
-        for (int b = off[1][e]; b < off[1][e + 1]; b++) tb[b] = off[0][e] + 2 * (b - off[1][e]);
+        for (int b = off[1][e]; b < off[1][e + 1]; b++) tb[b] = off[0][e] + block * (b - off[1][e]);
     }
     for (int t = off[0][E] + tid; t < max_tiles; t += blockDim.x) te[t] = -1;
     if (tid == 0) *n_tb = off[1][E];
 }
 
-/* Block of (token block, row block x): the token tiles t and, if it is the same expert's, t + 1, where t = tb[w / X].
-   act[32 t + token][32 x + row] = silu(gate . x) * (up . x): a wave's two weight tiles are the gate and the up rows of
-   the same 32 columns, so both halves of an output are in one lane. */
-template <int DT>
+/* The tiles of token block item / X: t = tb[item / X] and the next ones of its expert, up to two (FAST four), the last
+   one again past them. Returns how many there are. */
+template <bool FAST>
+__device__ __forceinline__ int gsx_tiles(const int* __restrict__ te, int t, int T, int (&tt)[2 * TG_T]) {
+    int n = 1;
+#pragma unroll
+    for (int j = 1; j < (FAST ? 4 : 2); j++) n += n == j && t + j < T && te[t + j] == te[t];
+#pragma unroll
+    for (int j = 0; j < 2 * TG_T; j++) tt[j] = t + min(j, n - 1);
+    return n;
+}
+
+/* Block of (token block, row block x). act[32 t + token][32 x + row] = silu(gate . x) * (up . x): a wave's two weight
+   tiles are the gate and the up rows of the same 32 columns, so both halves of an output are in one lane. */
+template <int DT, bool FAST>
 __global__ __launch_bounds__(TG_THREADS) void gsx_tile_in_kernel(qmat gate, qmat up, tg_images im, const int* __restrict__ te,
                                                                  const int* __restrict__ tb, const int* __restrict__ n_tb, int T,
                                                                  float inv, float* __restrict__ act) {
     __shared__ __attribute__((aligned(1024))) uint8_t lds[tg_lds<DT>::BYTES];
+    constexpr int NT = FAST ? 2 : 1;
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int H = gate.cols, I = gate.rows, X = I / 128, S0 = H / 256;
     const int item = tg_item(*n_tb * X);
     if (item < 0) return;
     const int t = tb[item / X], x = item - item / X * X, e = te[t];
-    const bool two = t + 1 < T && te[t + 1] == e;
+    int tt[2 * TG_T];
+    const int n = gsx_tiles<FAST>(te, t, T, tt);
     const int rg = wv & 3, tg = wv >> 2;
-    const int tt[TG_T] = {t, two ? t + 1 : t};
     const qmat& m = wv & 1 ? up : gate;
     const uint8_t* tile = m.tiled + ((size_t)e * (I / 32) + 4 * x + (wv >> 1)) * S0 * tg_lds<DT>::TB;
-    f32x16 acc[2] = {};
-    tg_body<DT>(tg_sources<DT>(im, tt, tile, S0, 0, wv), S0, lds, __builtin_amdgcn_readfirstlane(tg_lds_addr(lds)), wv, lane, 2 * rg, tg,
-                tg == 0 || two, acc);
-    if (tg && !two) return;
+    f32x16 acc[NT][2] = {};
+    tg_body<DT, FAST>(tg_sources<DT, FAST>(im, tt, tile, S0, wv), S0, lds, __builtin_amdgcn_readfirstlane(tg_lds_addr(lds)), wv, lane, 2 * rg,
+                      tg, NT * tg < n, acc);
     const int l32 = lane & 31, kq = lane >> 5;
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
-        const int tok = 8 * (r >> 2) + 4 * kq + (r & 3);
-        const float g = acc[0][r] * inv;
-        act[(size_t)(32 * (t + tg) + tok) * I + 32 * (4 * x + rg) + l32] = (g / (1.0f + expf(-g))) * (acc[1][r] * inv);
+    for (int j = 0; j < NT; j++) {
+        if (NT * tg + j >= n) break;
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const int tok = 8 * (r >> 2) + 4 * kq + (r & 3);
+            const float g = acc[j][0][r] * inv;
+            act[(size_t)(32 * (t + NT * tg + j) + tok) * I + 32 * (4 * x + rg) + l32] = (g / (1.0f + expf(-g))) * (acc[j][1][r] * inv);
+        }
     }
 }
 
 /* ypart[(row K + slot) H + n] = w_slot (down_e[n] . act[pair]) for the pairs of the block's token tiles. */
-template <int DT>
+template <int DT, bool FAST>
 __global__ __launch_bounds__(TG_THREADS) void gsx_tile_down_kernel(qmat down, tg_images im, const int* __restrict__ te,
                                                                    const int* __restrict__ tb, const int* __restrict__ n_tb, int T,
                                                                    const int* __restrict__ toff, const int* __restrict__ count,
@@ -464,31 +499,49 @@ __global__ __launch_bounds__(TG_THREADS) void gsx_tile_down_kernel(qmat down, tg
                                                                    const route_out* __restrict__ rt, int K, const float* __restrict__ inv,
                                                                    float* __restrict__ ypart) {
     __shared__ __attribute__((aligned(1024))) uint8_t lds[tg_lds<DT>::BYTES];
+    constexpr int NT = FAST ? 2 : 1;
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int H = down.rows, X = H / 256, S0 = down.cols / 256;
     const int item = tg_item(*n_tb * X);
     if (item < 0) return;
     const int t = tb[item / X], x = item - item / X * X, e = te[t];
-    const bool two = t + 1 < T && te[t + 1] == e;
+    int tt[2 * TG_T];
+    const int n = gsx_tiles<FAST>(te, t, T, tt);
     const int rg = wv & 3, tg = wv >> 2;
-    const int tt[TG_T] = {t, two ? t + 1 : t};
     const uint8_t* tile = down.tiled + ((size_t)e * (H / 32) + TG_R * x + wv) * S0 * tg_lds<DT>::TB;
-    f32x16 acc[2] = {};
-    tg_body<DT>(tg_sources<DT>(im, tt, tile, S0, 0, wv), S0, lds, __builtin_amdgcn_readfirstlane(tg_lds_addr(lds)), wv, lane, 2 * rg, tg,
-                tg == 0 || two, acc);
-    if (tg && !two) return;
-    const int l32 = lane & 31, kq = lane >> 5, j0 = 32 * (t + tg - toff[e]), c = count[e];
+    f32x16 acc[NT][2] = {};
+    tg_body<DT, FAST>(tg_sources<DT, FAST>(im, tt, tile, S0, wv), S0, lds, __builtin_amdgcn_readfirstlane(tg_lds_addr(lds)), wv, lane, 2 * rg,
+                      tg, NT * tg < n, acc);
+    const int l32 = lane & 31, kq = lane >> 5, c = count[e];
 #pragma unroll
-    for (int r = 0; r < 16; r++) {
-        const int j = j0 + 8 * (r >> 2) + 4 * kq + (r & 3);
-        if (j < c) {
-            const int p = pairs[(size_t)e * cap + j], row = p / ROUTE_K_MAX, slot = p % ROUTE_K_MAX;
-            const float wt = rt[row].weights[slot], f = inv[32 * (t + tg) + j - j0];
-            float* y = ypart + ((size_t)row * K + slot) * H + 32 * (TG_R * x + 2 * rg) + l32;
-            y[0] = wt * (acc[0][r] * f);
-            y[32] = wt * (acc[1][r] * f);
+    for (int i = 0; i < NT; i++) {
+        if (NT * tg + i >= n) break;
+        const int tile_t = t + NT * tg + i, j0 = 32 * (tile_t - toff[e]);
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+            const int j = j0 + 8 * (r >> 2) + 4 * kq + (r & 3);
+            if (j < c) {
+                const int p = pairs[(size_t)e * cap + j], row = p / ROUTE_K_MAX, slot = p % ROUTE_K_MAX;
+                const float wt = rt[row].weights[slot], f = inv[32 * tile_t + j - j0];
+                float* y = ypart + ((size_t)row * K + slot) * H + 32 * (TG_R * x + 2 * rg) + l32;
+                y[0] = wt * (acc[i][0][r] * f);
+                y[32] = wt * (acc[i][1][r] * f);
+            }
         }
     }
+}
+
+/* Columns 8 c8 .. of row `row` into the image: both pieces at img_put's place, or with fast the hi piece alone, at the
+   same place of an image of half the size. */
+__device__ __forceinline__ void gsx_put(u32x4* img, bool order_b, bool fast, int row, int K, int c8, const u32x4& vh, const u32x4& vl) {
+    if (!fast) {
+        img_put(order_b ? nullptr : img, order_b ? img : nullptr, row, K, c8, vh, vl);
+        return;
+    }
+    const int c = 8 * (c8 & 31), r = c & (order_b ? 127 : 63);
+    const int U = order_b ? 2 * (c >> 7) + ((r >> 5) & 1) : c >> 6, kq = order_b ? (r >> 3) & 1 : (r >> 4) & 1;
+    const int i = order_b ? ((r >> 4) & 1) + 2 * (r >> 6) : ((r >> 5) << 1) | ((r >> 3) & 1);
+    img[((size_t)(row >> 5) * (K / 256) + (c8 >> 5)) * 1024 + (U * 4 + i) * 64 + (row & 31) + 32 * kq] = vh;
 }
 
 /* The images (one column order) and, for Q4_K weights, group sums of the virtual token tiles: block (b, t) takes
@@ -496,7 +549,7 @@ __global__ __launch_bounds__(TG_THREADS) void gsx_tile_down_kernel(qmat down, tg
    again), row pair / ROUTE_K_MAX of x, times f (every row's values stay under 2^14). */
 __global__ __launch_bounds__(256) void gsx_image_kernel(const float* __restrict__ x, int K, float f, const int* __restrict__ pairs,
                                                         const int* __restrict__ count, int cap, const int* __restrict__ toff,
-                                                        const int* __restrict__ te, u32x4* __restrict__ imga, u32x4* __restrict__ imgb,
+                                                        const int* __restrict__ te, u32x4* __restrict__ img, bool order_b, bool fast,
                                                         _Float16* __restrict__ sums) {
     const int b = blockIdx.x, t = blockIdx.y;
     const int e = te[t];
@@ -511,9 +564,9 @@ __global__ __launch_bounds__(256) void gsx_image_kernel(const float* __restrict_
         const float ev[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
         u32x4 vh, vl;
         float sum;
-        th_split8(ev, f, vh, vl, sum);
-        img_put(imga, imgb, 32 * t + l, K, c8, vh, vl);
-        if (imgb) continue;
+        th_split8(ev, f, fast, vh, vl, sum);
+        gsx_put(img, order_b, fast, 32 * t + l, K, c8, vh, vl);
+        if (order_b) continue;
         const float t16 = sum + __shfl_xor(sum, 1, WAVE), t32 = t16 + __shfl_xor(t16, 2, WAVE);
         if (!(c8 & 3)) th_sum(sums + ((size_t)t * (K / 256) + b) * 512, l, (c8 & 31) >> 2, t32);
     }
@@ -521,8 +574,8 @@ __global__ __launch_bounds__(256) void gsx_image_kernel(const float* __restrict_
 
 /* The same of the SwiGLU output's rows (row 32 t + l of x for token l of tile t), each scaled by its own power of
    two, whose inverse goes to inv: block t, eight threads a row, the row read twice. */
-__global__ __launch_bounds__(256) void gsx_act_image_kernel(const float* __restrict__ x, int K, const int* __restrict__ te, u32x4* __restrict__ imga,
-                                                            u32x4* __restrict__ imgb, _Float16* __restrict__ sums, float* __restrict__ inv) {
+__global__ __launch_bounds__(256) void gsx_act_image_kernel(const float* __restrict__ x, int K, const int* __restrict__ te, u32x4* __restrict__ img,
+                                                            bool order_b, bool fast, _Float16* __restrict__ sums, float* __restrict__ inv) {
     const int t = blockIdx.x;
     if (te[t] < 0) return;
     const int l = threadIdx.x >> 3, j = threadIdx.x & 7, row = 32 * t + l;
@@ -542,14 +595,15 @@ __global__ __launch_bounds__(256) void gsx_act_image_kernel(const float* __restr
         const float ev[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
         u32x4 vh, vl;
         float sum;
-        th_split8(ev, f, vh, vl, sum);
-        img_put(imga, imgb, row, K, c, vh, vl);
-        if (imgb) continue;
+        th_split8(ev, f, fast, vh, vl, sum);
+        gsx_put(img, order_b, fast, row, K, c, vh, vl);
+        if (order_b) continue;
         const float t16 = sum + __shfl_xor(sum, 1, WAVE), t32 = t16 + __shfl_xor(t16, 2, WAVE);
         if (!(c & 3)) th_sum(sums + ((size_t)t * (K / 256) + (c >> 5)) * 512, l, (c & 31) >> 2, t32);
     }
 }
 
+template <bool FAST>
 static hipError_t launch_gsx_tiles(const gsx_args& a, bool in, hipStream_t s) {
     const qmat& m = in ? a.gate : a.down;
     const int X = in ? a.gate.rows / 128 : a.down.rows / 256, T = gsx_max_tiles(a.n, a.K, a.E);
@@ -558,13 +612,16 @@ static hipError_t launch_gsx_tiles(const gsx_args& a, bool in, hipStream_t s) {
     const int *tb = a.tb, *n_tb = a.tb + a.max_tiles;
     auto go = [&](auto dt) {
         constexpr int DT = decltype(dt)::value;
-        if (in) gsx_tile_in_kernel<DT><<<blocks, TG_THREADS, 0, s>>>(a.gate, a.up, k, a.te, tb, n_tb, T, 1.0f / a.xscale, a.act);
-        else gsx_tile_down_kernel<DT><<<blocks, TG_THREADS, 0, s>>>(a.down, k, a.te, tb, n_tb, T, a.toff, a.count, a.pairs, a.cap, a.rt, a.K, a.inv, a.ypart);
+        if (in) gsx_tile_in_kernel<DT, FAST><<<blocks, TG_THREADS, 0, s>>>(a.gate, a.up, k, a.te, tb, n_tb, T, 1.0f / a.xscale, a.act);
+        else gsx_tile_down_kernel<DT, FAST><<<blocks, TG_THREADS, 0, s>>>(a.down, k, a.te, tb, n_tb, T, a.toff, a.count, a.pairs, a.cap, a.rt, a.K, a.inv, a.ypart);
     };
     switch (m.dtype) {
     case VITNA_DTYPE_Q4_K: go(std::integral_constant<int, VITNA_DTYPE_Q4_K>()); break;
     case VITNA_DTYPE_Q6_K: go(std::integral_constant<int, VITNA_DTYPE_Q6_K>()); break;
-    default: go(std::integral_constant<int, VITNA_DTYPE_Q8_0>()); break;
+    default:
+        if constexpr (FAST) return hipErrorInvalidValue;
+        else go(std::integral_constant<int, VITNA_DTYPE_Q8_0>());
+        break;
     }
     return hipGetLastError();
 }
@@ -575,15 +632,14 @@ hipError_t launch_gsx(const gsx_args& a, hipStream_t s) {
         a.E < 1 || a.E > ROUTE_E_MAX || a.n < 1 || a.cap < a.n || a.max_tiles < gsx_max_tiles(a.n, a.K, a.E) || !(a.xscale > 0.0f))
         return hipErrorInvalidValue;
     const int H = a.gate.cols, I = a.gate.rows, T = gsx_max_tiles(a.n, a.K, a.E);
-    gsx_plan_kernel<<<1, 256, 0, s>>>(a.count, a.E, a.toff, a.te, T, a.tb, a.tb + a.max_tiles);
-    const bool in_b = a.gate.dtype == VITNA_DTYPE_Q6_K, dn_b = a.down.dtype == VITNA_DTYPE_Q6_K;
+    gsx_plan_kernel<<<1, 256, 0, s>>>(a.count, a.E, a.toff, a.te, T, a.fast ? 4 : 2, a.tb, a.tb + a.max_tiles);
     u32x4* ii = reinterpret_cast<u32x4*>(a.img_in);
     u32x4* ia = reinterpret_cast<u32x4*>(a.img_act);
     _Float16* sums = reinterpret_cast<_Float16*>(a.sums);
-    gsx_image_kernel<<<dim3(H / 256, T), 256, 0, s>>>(a.xn, H, a.xscale, a.pairs, a.count, a.cap, a.toff, a.te, in_b ? nullptr : ii,
-                                                      in_b ? ii : nullptr, sums);
-    hipError_t err = launch_gsx_tiles(a, true, s);
+    gsx_image_kernel<<<dim3(H / 256, T), 256, 0, s>>>(a.xn, H, a.xscale, a.pairs, a.count, a.cap, a.toff, a.te, ii,
+                                                      a.gate.dtype == VITNA_DTYPE_Q6_K, a.fast, sums);
+    hipError_t err = a.fast ? launch_gsx_tiles<true>(a, true, s) : launch_gsx_tiles<false>(a, true, s);
     if (err != hipSuccess) return err;
-    gsx_act_image_kernel<<<T, 256, 0, s>>>(a.act, I, a.te, dn_b ? nullptr : ia, dn_b ? ia : nullptr, sums, a.inv);
-    return launch_gsx_tiles(a, false, s);
+    gsx_act_image_kernel<<<T, 256, 0, s>>>(a.act, I, a.te, ia, a.down.dtype == VITNA_DTYPE_Q6_K, a.fast, sums, a.inv);
+    return a.fast ? launch_gsx_tiles<true>(a, false, s) : launch_gsx_tiles<false>(a, false, s);
 }

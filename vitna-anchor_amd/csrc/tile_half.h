@@ -47,8 +47,8 @@ __device__ __forceinline__ float th_scale(float largest) {
     return __uint_as_float((uint32_t)(min(max(13 - (e - 127), -100), 100) + 127) << 23);
 }
 
-/* eight values times f as f16 hi and lo in the operands' order, and the sum of hi + lo */
-__device__ __forceinline__ void th_split8(const float e[8], float f, u32x4& vh, u32x4& vl, float& sum) {
+/* eight values times f as f16 hi and lo in the operands' order, and the sum of hi + lo (fast: of hi) */
+__device__ __forceinline__ void th_split8(const float e[8], float f, bool fast, u32x4& vh, u32x4& vl, float& sum) {
     h8 h, l;
     float s = 0.0f;
 #pragma unroll
@@ -59,7 +59,7 @@ __device__ __forceinline__ void th_split8(const float e[8], float f, u32x4& vh, 
         const _Float16 b = (_Float16)(v - (float)a);
         h[at] = a;
         l[at] = b;
-        s += (float)a + (float)b;
+        s += fast ? (float)a : (float)a + (float)b;
     }
     vh = __builtin_bit_cast(u32x4, h);
     vl = __builtin_bit_cast(u32x4, l);

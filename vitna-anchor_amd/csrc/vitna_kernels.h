@@ -322,6 +322,7 @@ struct gsx_args {
     const int* count;      /* [E] */
     const int* pairs;      /* [E][cap] */
     int E, K, cap, n;
+    bool fast;             /* --precision fast: activations in f16 alone, one product a weight */
     int *toff, *te;        /* [E + 1], [max_tiles] */
     int* tb;               /* [max_tiles + 1]: the first tile of each token block, then the number of blocks */
     int max_tiles;         /* at least gsx_max_tiles(n, K, E) */
@@ -335,7 +336,7 @@ struct gsx_args {
 };
 bool gsx_fits(const qmat& gate, const qmat& up, const qmat& down);
 int gsx_max_tiles(int n, int K, int E);
-/* Token blocks of the grouped experts: two tiles of one expert each (kernels_tgemm.hip). */
+/* The most token blocks of the grouped experts: two tiles (a fast pass: four) of one expert each. */
 int gsx_max_blocks(int n, int K, int E);
 size_t gsx_tiled_bytes(const qmat& m, int n_experts);
 hipError_t launch_gsx_tile(const qmat& m, int n_experts, uint8_t* dst, hipStream_t s);
