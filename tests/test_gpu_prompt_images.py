@@ -1,0 +1,42 @@
+"""A prompt pass's attention from the chunks' images (eight row tiles or more) against the same rows in passes of fewer
+tiles, whose blocks split the chunks themselves: the same bits of every row's attention output, for passes that start
+before, on and after a 64-position chunk's edge, with a last tile part-filled, at 8, 4 and 1 query heads a kv head.
+One layer, so that the rows' queries, keys and values are the same bits however the pass is cut.
+"""
+import numpy as np
+import pytest
+
+import vitna_amd as va
+from test_gpu_decode import say
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("heads,kvs", [(16, 2), (8, 2), (2, 2)])
+@pytest.mark.parametrize("start,n", [(0, 520), (63, 513), (64, 577), (190, 600)])
+def test_images_against_own_split(heads, kvs, start, n):
+    say("prompt images", heads, kvs, "rows", start, n)
+    model = va.Model(va.shape(n_layers=1, hidden=512, intermediate=256, n_heads=heads, n_kv_heads=kvs, head_dim=128, vocab=1000, n_experts=16,
+                              n_experts_used=4, norm_std=0.1, ctx=start + n, seqs=1), 1357)
+    a, b = va.Device(model), va.Device(model)
+    try:
+        kd = kvs * 128
+        k, v = va.normal(3, 1, start * kd + 1)[:start * kd].reshape(start, kd), va.normal(3, 2, start * kd + 1)[:start * kd].reshape(start, kd)
+        for d in (a, b):
+            if start:
+                d.kv(0, 0, 0, start, k, v)
+        rows = [((13 * i + 5) % 1000, start + i, 0) for i in range(n)]
+        a.rows_step(rows, logits=False)
+        piece = 7 * 4 * (16 // (heads // kvs))  # seven tiles
+        for at in range(0, n, piece):
+            some = rows[at:at + piece]
+            b.rows_step(some, logits=False)
+            if len(some) == 1:
+                continue  # a single row takes the decode kernels
+            for i in range(0, len(some), 5):
+                got, want = a.attention_io(at + i)[1], b.attention_io(i)[1]
+                assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), ("row", at + i)
+    finally:
+        a.close()
+        b.close()
+        model.free()

@@ -2110,6 +2110,7 @@ static hipError_t enqueue_rows_attention(vitna_cuda_model* g, int layer, int n, 
     a.rows = g->rows_dev;
     a.n_rows = n;
     a.partial = g->partial;
+    a.partial_rows = ROWS_MAX;
     a.att = g->att;
     a.n_heads = g->nh; a.n_kv = g->nkv; a.hd = g->hd; a.ctx = g->ctx; a.splits_max = g->splits_max;
     a.splits_grid = g->splits_grid;

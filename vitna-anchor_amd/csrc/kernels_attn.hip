@@ -547,9 +547,7 @@ hipError_t launch_attention(const attn_args& a, hipStream_t s) {
    RW = 16 / G rows of the tile times the G heads, against the chunk's 64 positions, each row masked to the
    positions up to its own. The queries come prepared (launch_attention_prepare). The scores of each chunk fold
    into a running maximum and sum per column, the values into O rescaled as the maximum grows, and the block
-   writes att itself (O / sum): no chunk leaves a partial and no merge runs. A chunk's keys and values are
-   requested before the barrier that frees the LDS of the previous one; the other block of the CU covers the
-   wait. Passes of more than 64 rows reach it (the exact-rows limit), so it is held to 1e-3, not to a step's
+   writes att itself (O / sum): no chunk leaves a partial and no merge runs. Passes of more than 64 rows reach it (the exact-rows limit), so it is held to 1e-3, not to a step's
    bits.
 
    The products run on the bf16 matrix cores. Each operand is split into bf16 hi + lo (lo the rounding of what hi
@@ -577,7 +575,96 @@ __device__ __forceinline__ void fl_split4(float x0, float x1, float x2, float x3
 __device__ __forceinline__ fl_bf8 fl_join(uint2 a, uint2 b) { return __builtin_bit_cast(fl_bf8, u32x4{a.x, a.y, b.x, b.y}); }
 #define FL_MMA(A, B, C) __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B, C, 0, 0, 0)
 
-template <int G>
+#define FL_K (64 * 64)  /* dwords of a chunk's keys, hi or lo: [position][16 pieces of 8 dimensions] */
+#define FL_V (128 * 32) /* of its values: [dimension][16 pieces of 4 positions] */
+#define FL_IMAGE (2 * (FL_K + FL_V)) /* a chunk's image: keys hi, lo, values hi, lo */
+
+/* A thread's share of a chunk: positions 32 (i / 4) + 4 pg + i % 4, dimensions 4 cc .. 4 cc + 3 (a wave's load is two
+   whole 512-byte rows); zeros past position last. */
+struct fl_share {
+    float4 k[8], v[8];
+};
+__device__ __forceinline__ void fl_fetch(const float* kc, const float* vc, int kv_dim, int h, int t0, int last, fl_share& f) {
+    const int pg = threadIdx.x >> 5, cc = threadIdx.x & 31;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const int p = 32 * (i >> 2) + 4 * pg + (i & 3), pos = t0 + p;
+        const bool ok = pos <= last;
+        const size_t at = (size_t)(ok ? pos : 0) * kv_dim + (size_t)h * 128 + 4 * cc;
+        f.k[i] = ok ? *reinterpret_cast<const float4*>(kc + at) : make_float4(0.f, 0.f, 0.f, 0.f);
+        f.v[i] = ok ? *reinterpret_cast<const float4*>(vc + at) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+}
+/* and where it goes, split, in the chunk's keys sk and values sv */
+__device__ __forceinline__ void fl_store(const fl_share& f, uint32_t* sk, uint32_t* sv) {
+    const int pg = threadIdx.x >> 5, cc = threadIdx.x & 31;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const int p = 32 * (i >> 2) + 4 * pg + (i & 3);
+        uint2 hh, ll;
+        fl_split4(f.k[i].x, f.k[i].y, f.k[i].z, f.k[i].w, hh, ll);
+        const int ka = (p * 16 + ((cc >> 1) ^ (p & 15))) * 4 + 2 * (cc & 1);
+        *reinterpret_cast<uint2*>(&sk[ka]) = hh;
+        *reinterpret_cast<uint2*>(&sk[FL_K + ka]) = ll;
+    }
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        const int pc = 8 * q + pg; /* the piece of positions 32 q + 4 pg .. + 3 */
+#pragma unroll
+        for (int d = 0; d < 4; d++) {
+            const float4* v = f.v + 4 * q;
+            const float x0 = d == 0 ? v[0].x : d == 1 ? v[0].y : d == 2 ? v[0].z : v[0].w;
+            const float x1 = d == 0 ? v[1].x : d == 1 ? v[1].y : d == 2 ? v[1].z : v[1].w;
+            const float x2 = d == 0 ? v[2].x : d == 1 ? v[2].y : d == 2 ? v[2].z : v[2].w;
+            const float x3 = d == 0 ? v[3].x : d == 1 ? v[3].y : d == 2 ? v[3].z : v[3].w;
+            uint2 hh, ll;
+            fl_split4(x0, x1, x2, x3, hh, ll);
+            const int dim = 4 * cc + d, va = (dim * 16 + (pc ^ (dim & 15))) * 2;
+            *reinterpret_cast<uint2*>(&sv[va]) = hh;
+            *reinterpret_cast<uint2*>(&sv[FL_V + va]) = ll;
+        }
+    }
+}
+
+/* The images of the pass's whole chunks (every position written), for passes of many tiles: splitting a chunk is about
+   as much VALU work as its products are matrix work, and a tile's block that splits its own repeats it in every
+   tile. Block (kv head, chunk); images at [kv head][splits_max] of a.partial, which such a pass has no other use
+   for. A 1024-row pass at positions 1024 .. 2047 (32 query, 4 kv heads; kernel trace)
+   178 -> 126 us and 8 for the images, at 3072 .. 4095 364 -> 252 and 11. */
+__global__ __launch_bounds__(256) void attention_image_kernel(attn_args a) {
+    __shared__ int most[4];
+    const int tid = threadIdx.x, h = blockIdx.x, c = blockIdx.y;
+    int pmax = 0;
+    for (int r = tid; r < a.n_rows; r += 256) pmax = max(pmax, a.rows[r].pos);
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) pmax = max(pmax, __shfl_xor(pmax, d, WAVE));
+    if ((tid & 63) == 0) most[tid >> 6] = pmax;
+    __syncthreads();
+    pmax = max(max(most[0], most[1]), max(most[2], most[3]));
+    if (c >= pmax / ATTN_CHUNK) return;
+    const size_t seq = (size_t)a.rows[0].seq * a.seq_stride;
+    fl_share f;
+    fl_fetch(a.k_cache + seq, a.v_cache + seq, a.n_kv * 128, h, c * ATTN_CHUNK, pmax, f);
+    uint32_t* out = reinterpret_cast<uint32_t*>(a.partial) + ((size_t)h * a.splits_max + c) * FL_IMAGE;
+    fl_store(f, out, out + 2 * FL_K);
+}
+
+/* A wave's quarter of n KB from src to LDS (lane l's 16 bytes at + 16 l), waited for by fl_wait; the compiler does not
+   count these loads, and M0 is set nowhere else here. */
+template <int KB>
+__device__ __forceinline__ void fl_load(const uint32_t* src, uint32_t lds, int wave, int lane) {
+#pragma unroll
+    for (int j = 0; j < KB / 4; j++)
+        asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(16 * lane), "s"(src + (4 * j + wave) * 256),
+                     "s"(lds + (4 * j + wave) * 1024)
+                     : "memory", "m0");
+}
+__device__ __forceinline__ void fl_wait() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+/* IMAGED: attention_image_kernel ran; a tile's whole chunks come from their images (the keys of the next chunk while
+   the values of this one are multiplied, and the other way round), its last chunk is split here, zeros past the tile's
+   last position. Both forms multiply the same values in the same order. */
+template <int G, bool IMAGED>
 __global__ __launch_bounds__(256, 2) void attention_flash_kernel(attn_args a) {
     constexpr int HD = 128, RW = 16 / G, TQ = 4 * RW;
     /* a tile's work grows with its position; the second half of the grid takes the tiles in reverse, so the two
@@ -593,9 +680,7 @@ __global__ __launch_bounds__(256, 2) void attention_flash_kernel(attn_args a) {
     const int seq = a.rows[r_first].seq, kv_dim = a.n_kv * HD;
     const float* kc = a.k_cache + (size_t)seq * a.seq_stride;
     const float* vc = a.v_cache + (size_t)seq * a.seq_stride;
-    /* keys [position][16 chunks of 8 dimensions], values [dimension][16 chunks of 4 positions], hi and lo */
-    __shared__ __attribute__((aligned(16))) uint32_t skh[64 * 64], skl[64 * 64];
-    __shared__ __attribute__((aligned(16))) uint32_t svh[128 * 32], svl[128 * 32];
+    __shared__ __attribute__((aligned(1024))) uint32_t sk[2 * FL_K], sv[2 * FL_V];
 
     const int rr = r_first + wave * RW + c16 / G, g = c16 % G;
     const bool colv = rr < r_end;
@@ -617,57 +702,12 @@ __global__ __launch_bounds__(256, 2) void attention_flash_kernel(attn_args a) {
             ql[s] = fl_join(l0, l1);
         }
     }
-    /* a thread's fetch: positions 32 (i / 4) + 4 pg + i % 4 of the chunk, dimensions 4 cc .. 4 cc + 3 (a wave's
-       load is two whole 512-byte rows) */
-    const int pg = tid >> 5, cc = tid & 31;
-    float4 kr[8], vr[8];
-    auto fetch = [&](int c) {
-        const int t0 = c * ATTN_CHUNK;
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int p = 32 * (i >> 2) + 4 * pg + (i & 3), pos = t0 + p;
-            const bool ok = pos <= pmax;
-            const size_t at = (size_t)(ok ? pos : 0) * kv_dim + (size_t)h * HD + 4 * cc;
-            kr[i] = ok ? *reinterpret_cast<const float4*>(kc + at) : make_float4(0.f, 0.f, 0.f, 0.f);
-            vr[i] = ok ? *reinterpret_cast<const float4*>(vc + at) : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-    };
     float m_run = -INFINITY, l_run = 0.0f;
-    at_f4 O[8];
+    at_f4 O[8], S[4];
 #pragma unroll
     for (int j = 0; j < 8; j++) O[j] = at_f4{0.f, 0.f, 0.f, 0.f};
-    for (int c = 0; c < nch; c++) {
-        fetch(c);
-        __syncthreads(); /* the previous chunk's fragment reads are done */
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            const int p = 32 * (i >> 2) + 4 * pg + (i & 3);
-            uint2 hh, ll;
-            fl_split4(kr[i].x, kr[i].y, kr[i].z, kr[i].w, hh, ll);
-            const int ka = (p * 16 + ((cc >> 1) ^ (p & 15))) * 4 + 2 * (cc & 1);
-            *reinterpret_cast<uint2*>(&skh[ka]) = hh;
-            *reinterpret_cast<uint2*>(&skl[ka]) = ll;
-        }
-#pragma unroll
-        for (int q = 0; q < 2; q++) {
-            const int pc = 8 * q + pg; /* the chunk of positions 32 q + 4 pg .. + 3 */
-#pragma unroll
-            for (int d = 0; d < 4; d++) {
-                const float4 *v = vr + 4 * q;
-                const float x0 = d == 0 ? v[0].x : d == 1 ? v[0].y : d == 2 ? v[0].z : v[0].w;
-                const float x1 = d == 0 ? v[1].x : d == 1 ? v[1].y : d == 2 ? v[1].z : v[1].w;
-                const float x2 = d == 0 ? v[2].x : d == 1 ? v[2].y : d == 2 ? v[2].z : v[2].w;
-                const float x3 = d == 0 ? v[3].x : d == 1 ? v[3].y : d == 2 ? v[3].z : v[3].w;
-                uint2 hh, ll;
-                fl_split4(x0, x1, x2, x3, hh, ll);
-                const int dim = 4 * cc + d, va = (dim * 16 + (pc ^ (dim & 15))) * 2;
-                *reinterpret_cast<uint2*>(&svh[va]) = hh;
-                *reinterpret_cast<uint2*>(&svl[va]) = ll;
-            }
-        }
-        __syncthreads();
-        const int t0 = c * ATTN_CHUNK;
-        at_f4 S[4];
+    /* a chunk's scores into S as weights, O rescaled */
+    auto scores = [&](int t0) {
 #pragma unroll
         for (int pt = 0; pt < 4; pt++) {
             const int p = 16 * pt + c16;
@@ -675,8 +715,8 @@ __global__ __launch_bounds__(256, 2) void attention_flash_kernel(attn_args a) {
 #pragma unroll
             for (int s = 0; s < 4; s++) {
                 const int ka = (p * 16 + ((4 * s + kq) ^ (p & 15))) * 4;
-                const fl_bf8 kh = *reinterpret_cast<const fl_bf8*>(&skh[ka]);
-                const fl_bf8 kl = *reinterpret_cast<const fl_bf8*>(&skl[ka]);
+                const fl_bf8 kh = *reinterpret_cast<const fl_bf8*>(&sk[ka]);
+                const fl_bf8 kl = *reinterpret_cast<const fl_bf8*>(&sk[FL_K + ka]);
                 acc = FL_MMA(kh, qh[s], acc);
                 acc = FL_MMA(kh, ql[s], acc);
                 acc = FL_MMA(kl, qh[s], acc);
@@ -714,6 +754,8 @@ __global__ __launch_bounds__(256, 2) void attention_flash_kernel(attn_args a) {
         for (int j = 0; j < 8; j++)
 #pragma unroll
             for (int i = 0; i < 4; i++) O[j][i] *= fo[i];
+    };
+    auto values = [&]() {
 #pragma unroll
         for (int s = 0; s < 2; s++) {
             uint2 ph0, pl0, ph1, pl1;
@@ -725,13 +767,39 @@ __global__ __launch_bounds__(256, 2) void attention_flash_kernel(attn_args a) {
                 const int dim = 16 * j + c16;
                 const int va0 = (dim * 16 + ((8 * s + kq) ^ (dim & 15))) * 2;
                 const int va1 = (dim * 16 + ((8 * s + 4 + kq) ^ (dim & 15))) * 2;
-                const fl_bf8 vh = fl_join(*reinterpret_cast<const uint2*>(&svh[va0]), *reinterpret_cast<const uint2*>(&svh[va1]));
-                const fl_bf8 vl = fl_join(*reinterpret_cast<const uint2*>(&svl[va0]), *reinterpret_cast<const uint2*>(&svl[va1]));
+                const fl_bf8 vh = fl_join(*reinterpret_cast<const uint2*>(&sv[va0]), *reinterpret_cast<const uint2*>(&sv[va1]));
+                const fl_bf8 vl = fl_join(*reinterpret_cast<const uint2*>(&sv[FL_V + va0]), *reinterpret_cast<const uint2*>(&sv[FL_V + va1]));
                 O[j] = FL_MMA(ph, vh, O[j]);
                 O[j] = FL_MMA(ph, vl, O[j]);
                 O[j] = FL_MMA(pl, vh, O[j]);
             }
         }
+    };
+    int c = 0;
+    if constexpr (IMAGED) {
+        const int w = __builtin_amdgcn_readfirstlane(wave);
+        auto lds = [](const void* p) { return (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(__attribute__((address_space(3))) const uint8_t*)p); };
+        const uint32_t ks = lds(sk), vs = lds(sv);
+        const uint32_t* img = reinterpret_cast<const uint32_t*>(a.partial) + (size_t)h * a.splits_max * FL_IMAGE;
+        const int whole = nch - 1;
+        if (whole) fl_load<32>(img, ks, w, lane);
+        for (; c < whole; c++) {
+            fl_wait(); /* the keys; every wave is past the values before */
+            fl_load<32>(img + (size_t)c * FL_IMAGE + 2 * FL_K, vs, w, lane);
+            scores(c * ATTN_CHUNK);
+            fl_wait(); /* the values; every wave is past the keys */
+            if (c + 1 < whole) fl_load<32>(img + (size_t)(c + 1) * FL_IMAGE, ks, w, lane);
+            values();
+        }
+    }
+    for (; c < nch; c++) {
+        fl_share f;
+        fl_fetch(kc, vc, kv_dim, h, c * ATTN_CHUNK, pmax, f);
+        __syncthreads(); /* the previous chunk's fragment reads are done */
+        fl_store(f, sk, sv);
+        __syncthreads();
+        scores(c * ATTN_CHUNK);
+        values();
     }
     /* att = O / sum: column 4 kq + i of the lane's O, dimension 16 j + c16 */
 #pragma unroll
@@ -746,15 +814,27 @@ __global__ __launch_bounds__(256, 2) void attention_flash_kernel(attn_args a) {
     }
 }
 
+/* Row tiles from which the chunks' images pay. 42 tiles of 333 rows from position 0 (at most 6 chunks) took 33.1 us
+   splitting their own and 26.5 + 5.4 with images, and the more chunks, the more there is to repeat; below eight tiles a
+   launch is a larger share than what is repeated. */
+#define FL_IMAGE_TILES 8
+
 hipError_t launch_attention_flash(const attn_args& a, hipStream_t s) {
     if (!attention_run_fits(a) || a.n_rows < 1) return hipErrorInvalidValue;
     const int G = a.n_heads / a.n_kv, tq = 4 * (16 / G);
     const dim3 grid(a.n_kv, (a.n_rows + tq - 1) / tq);
-    switch (G) {
-        case 8: attention_flash_kernel<8><<<grid, 256, 0, s>>>(a); break;
-        case 4: attention_flash_kernel<4><<<grid, 256, 0, s>>>(a); break;
-        case 2: attention_flash_kernel<2><<<grid, 256, 0, s>>>(a); break;
-        case 1: attention_flash_kernel<1><<<grid, 256, 0, s>>>(a); break;
+    /* (a.partial holds n_rows x n_heads x splits_max x (hd + 4) floats or more: a chunk's image takes 128 rows of one head) */
+    const bool imaged = (int)grid.y >= FL_IMAGE_TILES && (size_t)a.partial_rows * a.n_heads * (a.hd + 4) >= (size_t)a.n_kv * FL_IMAGE;
+    if (imaged) attention_image_kernel<<<dim3(a.n_kv, a.splits_grid > 0 ? a.splits_grid : a.splits_max), 256, 0, s>>>(a);
+    switch (imaged ? G : -G) {
+        case 8: attention_flash_kernel<8, true><<<grid, 256, 0, s>>>(a); break;
+        case 4: attention_flash_kernel<4, true><<<grid, 256, 0, s>>>(a); break;
+        case 2: attention_flash_kernel<2, true><<<grid, 256, 0, s>>>(a); break;
+        case 1: attention_flash_kernel<1, true><<<grid, 256, 0, s>>>(a); break;
+        case -8: attention_flash_kernel<8, false><<<grid, 256, 0, s>>>(a); break;
+        case -4: attention_flash_kernel<4, false><<<grid, 256, 0, s>>>(a); break;
+        case -2: attention_flash_kernel<2, false><<<grid, 256, 0, s>>>(a); break;
+        case -1: attention_flash_kernel<1, false><<<grid, 256, 0, s>>>(a); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

@@ -193,6 +193,7 @@ struct attn_args {
     const row_rec* rows;   /* device, n_rows */
     int n_rows;
     float* partial;        /* [n_rows][n_kv][splits_max][G][hd + 4]: values, max, sum, padding */
+    int partial_rows;      /* the rows partial was made for */
     float* att;            /* [n_rows][n_heads * hd] */
     int n_heads, n_kv, hd, ctx, splits_max;
     /* chunks the launch covers (the grid's first dimension): at least the most any row of the pass has, at most
