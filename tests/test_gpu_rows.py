@@ -251,6 +251,32 @@ def test_rows_projections_token_tiles(name):
         model.free()
 
 
+@pytest.mark.parametrize("n", [1, 31, 64, 65, 97, 200])
+def test_rows_projections_split_width(n):
+    """Matrices wider than 2048 columns split across blocks, whose sums the last block of a tile adds or, from three
+    token tiles (65 rows), a kernel of their own: row counts at the edges of the tiles and of the two, against
+    float64 within the 2e-5 of the bf16 pair, and the last 16 rows bit for bit as by themselves (a row's sums know
+    nothing of the others)."""
+    say("rows projections, split width", n)
+    model = va.Model(va.shape(**dict(WIDE, seqs=1)), 2718)
+    dev = va.Device(model)
+    try:
+        rng = np.random.RandomState(n)
+        for which in range(5):
+            mat = _matrix(model, 0, which)
+            W = oracle.widen(mat.bytes(), mat.dtype, mat.rows * mat.cols).reshape(mat.rows, mat.cols).astype(np.float64)
+            x = rng.standard_normal((n, mat.cols)).astype(np.float32)
+            y = dev.rows_project(0, which, x)
+            ref = x.astype(np.float64) @ W.T
+            assert float(np.max(np.abs(y - ref)) / np.max(np.abs(ref))) <= 2e-5, which
+            if n > 16:
+                part = dev.rows_project(0, which, x[n - 16:])
+                assert np.array_equal(y[n - 16:].view(np.uint32), part.view(np.uint32)), which
+    finally:
+        dev.close()
+        model.free()
+
+
 NARROW = dict(n_layers=2, hidden=256, intermediate=256, n_heads=2, n_kv_heads=1, head_dim=64, vocab=300, n_experts=8,
               n_experts_used=2, renormalize=0, rms_eps=1e-5, rope_theta=10000.0, dt_gate_up=va.Q8_0, dt_down=va.Q8_0,
               dt_q=va.Q8_0, dt_k=va.Q8_0, dt_v=va.Q8_0, dt_o=va.Q8_0, dt_head=va.Q8_0, dt_embed=va.Q8_0, norm_std=0.1,

@@ -382,7 +382,8 @@ __device__ __forceinline__ void sx_superblock(const skinny_args& a, const qmat& 
  * 8 split + v. The waves' sums are added through LDS in wave order. A matrix wider than 8 superblocks takes
  * several splits: each block stores its tile's sum in part[], and the block that finishes a tile last (its
  * counter in cnt[]) adds the splits' sums in split order, writes the result and clears the counter, so the
- * result does not depend on which block finishes last.
+ * result does not depend on which block finishes last. With a.fold (many token tiles) each split's block writes
+ * its sums to its own copy of y and skinny_fold_kernel adds them, in the same order.
  */
 template <int NT, int NR>
 __global__ __launch_bounds__(512) void skinny_exact_kernel(skinny_args a) {
@@ -391,11 +392,13 @@ __global__ __launch_bounds__(512) void skinny_exact_kernel(skinny_args a) {
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, KS = blockDim.x >> 6;
     const int l32 = lane & 31, kq = lane >> 5;
     int bx = blockIdx.x, mi = 0, tile0 = 0;
+    size_t fold0 = 0; /* with a.fold: the matrix's first copy in part */
     for (; mi < a.nm - 1; mi++) {
         const int nb = ((a.w[mi].rows + 31) / 32 + NR - 1) / NR * a.splits[mi];
         if (bx < nb) break;
         bx -= nb;
         tile0 += (a.w[mi].rows + 31) / 32;
+        fold0 += (size_t)a.splits[mi] * a.n * a.w[mi].rows;
     }
     const qmat& w = a.w[mi];
     const int splits = a.splits[mi], sp = bx % splits, tile = bx / splits * NR;
@@ -452,6 +455,16 @@ __global__ __launch_bounds__(512) void skinny_exact_kernel(skinny_args a) {
                 }
                 continue;
             }
+            if (a.fold) {
+                float* o = a.part + fold0 + (size_t)sp * a.n * w.rows + row0 + l32;
+                for (int r = wv; r < 16; r += KS) {
+                    float v = 0.0f;
+                    for (int u = 0; u < KS; u++) v += red[(u * 16 + r) * 64 + lane];
+                    const int tk = tok0 + 8 * (r >> 2) + 4 * kq + (r & 3);
+                    if (row0 + l32 < w.rows && tk < a.n) o[(size_t)tk * w.rows] = v;
+                }
+                continue;
+            }
             /* several splits: this block's sum of the tile into part[], then the last block of the tile adds them */
             const size_t slot = (size_t)tt * a.tiles + tile0 + tile + wr; /* the tile's counter */
             float* part = a.part + slot * a.split_max * 1024;
@@ -479,6 +492,32 @@ __global__ __launch_bounds__(512) void skinny_exact_kernel(skinny_args a) {
         }
     }
 }
+
+/* y (+)= the splits' sums, in split order, four values a thread */
+__global__ __launch_bounds__(256) void skinny_fold_kernel(const float* __restrict__ part, int splits, size_t n, float* __restrict__ y, int add) {
+    const size_t i0 = (size_t)blockIdx.x * 1024 + threadIdx.x;
+    float old[4], v[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        old[j] = add && i0 + 256 * j < n ? y[i0 + 256 * j] : 0.0f;
+        v[j] = 0.0f;
+    }
+    for (int u = 0; u < splits; u++)
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (i0 + 256 * j < n) v[j] += part[u * n + i0 + 256 * j];
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+        if (i0 + 256 * j < n) y[i0 + 256 * j] = add ? old[j] + v[j] : v[j];
+}
+
+/* Token tiles from which a split width's sums are added by skinny_fold_kernel. A tile's counter costs no launch, but
+   each count is a release and an acquire at agent scope, which write back and invalidate an XCD's L2: with few tiles
+   that hides behind the weights' reads, with many it is most of the time. A 4096-wide projection to 2048 (kernel
+   trace, us), with the counters, and the kernel + the fold: 1024 rows 152, 65 + 5; 333 rows 56, 26 + 4; 128 rows 20,
+   10 + 4; 96 rows 21, 12 + 4; 64 rows 12.3, 8 + 4; 32 rows 10.3, 6.5 + 2.5; 8 rows 9.8, 7 + 3: up to two tiles they
+   are level in the trace, and a pass of 8 rows 562 and 567 us, of 32 rows 2.50 and 2.53 ms (the launch's gap). */
+#define SK_FOLD_TILES 3
 
 /* ---- wide matrices (the LM head): activations staged in LDS ---------------- */
 
@@ -615,6 +654,7 @@ static hipError_t launch_skinny_exact(const skinny_args& a0, hipStream_t s) {
     }
     if (split_max > 1 && (!a.part || !a.cnt || (size_t)mt * tiles > a.cnt_cap || (size_t)mt * tiles * split_max * 1024 > a.part_cap))
         return hipErrorInvalidValue;
+    a.fold = split_max > 1 && mt >= SK_FOLD_TILES;
     /* many token tiles (a prompt's chunk): each block takes SK_NT of them, the weights loaded once for all, or
        two weight tiles against the same token tile, each unit's activations loaded once for both */
     const size_t lds = (size_t)ks * 16 * 64 * sizeof(float);
@@ -630,6 +670,12 @@ static hipError_t launch_skinny_exact(const skinny_args& a0, hipStream_t s) {
         }
     } else {
         skinny_exact_kernel<1, 1><<<dim3(blocks, mt), 64 * ks, lds, s>>>(a);
+    }
+    const float* part = a.part;
+    for (int i = 0; a.fold && i < a.nm; i++) {
+        const size_t y = (size_t)a.n * a.w[i].rows;
+        skinny_fold_kernel<<<(unsigned)((y + 1023) / 1024), 256, 0, s>>>(part, a.splits[i], y, a.y[i], a.add);
+        part += a.splits[i] * y;
     }
     return hipGetLastError();
 }

@@ -273,11 +273,12 @@ struct skinny_args {
     const uint32_t *s32, *s16;
     int n, add;
     /* matrices wider than 2048 columns split across blocks: part (part_cap floats) holds each split's sum of a
-       tile and cnt (cnt_cap ints, zero before the first call, left zero by every call) counts finished splits */
+       tile and cnt (cnt_cap ints, zero before the first call, left zero by every call) counts finished splits;
+       with fold, each split's copy of y instead, which a kernel of its own adds up */
     float* part;
     int* cnt;
     size_t part_cap, cnt_cap;
-    int splits[3], tiles, split_max; /* set by launch_skinny */
+    int splits[3], tiles, split_max, fold; /* set by launch_skinny */
 };
 hipError_t launch_split_rows(const float* x, int n, int K, int xstride, uint16_t* xh, uint16_t* xl, uint32_t* const* img,
                              hipStream_t s);
