@@ -237,6 +237,10 @@ const float* vitna_hip_logits_device(struct vitna_cuda_model* g);
     prefill grouping: model_cuda.cu:5151-5176, :2288-2343. Q8_0 experts. */
 bool vitna_hip_moe_prefill(struct vitna_cuda_model* g, size_t layer, float* x, size_t n, int32_t* chosen, char* err, size_t err_len);
 
+/** vitna_hip_moe_prefill with the result in out (n x hidden, which may be x). */
+bool vitna_hip_moe_prefill_to(struct vitna_cuda_model* g, size_t layer, const float* x, size_t n, float* out, int32_t* chosen,
+                              char* err, size_t err_len);
+
 /** vitna_hip_moe_prefill without allocating: no reference counterpart; for
     callers that cannot allocate device memory (code under HIP graph capture,
     tight serving loops, harnesses that forbid hipMalloc). x (n x hidden fp32)

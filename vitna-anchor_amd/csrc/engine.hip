@@ -19,6 +19,7 @@
 #include "vitna_kernels.h"
 #include "step_kernel.h"
 #include "expert_cache.h"
+#include "host_copy.h"
 #include "../../include/vitna_hip.h"
 
 #include <stdarg.h>
@@ -98,6 +99,7 @@ struct vitna_cuda_model {
     row_rec* rows_dev;
     row_rec* rows_host; /* pinned */
     hipEvent_t rows_copied;
+    host_copy* results; /* logits and prefilled rows into the caller's memory */
     bool row_set;       /* rows_dev[0] holds row_last (set_row); another pass of rows clears it */
     row_rec row_last;
     route_out* rt_host; /* pinned, ROWS_MAX: the routing a caller gives, on its way to rt */
@@ -118,6 +120,8 @@ struct vitna_cuda_model {
     uint32_t *gsx_img_in, *gsx_img_act;
     uint16_t* gsx_sums;
     float *gsx_act, *gsx_inv;
+    std::vector<uint64_t> seq_seen; /* by sequence: the last pass (seq_pass) that had a row of it */
+    uint64_t seq_pass;
     bool rows_shared_seq;       /* the pass's rows include two of one sequence (attention prepares first) */
     bool rows_one_seq;          /* every row of the pass is of one sequence (a prompt's chunk: tiles of rows) */
     /* the rows step's captured graphs, a few kept (least recently used replaced): one a pass shape */
@@ -512,6 +516,7 @@ extern "C" void vitna_cuda_free(struct vitna_cuda_model* g) {
     if (g->rt_host) (void)hipHostFree(g->rt_host);
     if (g->rt_copied) (void)hipEventDestroy(g->rt_copied);
     ec_destroy(g->ec);
+    host_copy_destroy(g->results);
     if (g->stream) (void)hipStreamDestroy(g->stream);
     delete g;
 }
@@ -683,7 +688,9 @@ extern "C" struct vitna_cuda_model* vitna_cuda_create(const vitna_llama_t* m, co
         fail(err, err_len, "clearing device scratch failed");
         return bail();
     }
-    if (hipHostMalloc((void**)&g->rows_host, R * sizeof(row_rec), 0) != hipSuccess ||
+    g->seq_seen.resize(m->seqs);
+    g->results = host_copy_create();
+    if (!g->results || hipHostMalloc((void**)&g->rows_host, R * sizeof(row_rec), 0) != hipSuccess ||
         hipHostMalloc((void**)&g->h_logits, 2 * R * E * 4, 0) != hipSuccess ||
         hipHostMalloc((void**)&g->rt_host, R * sizeof(route_out), 0) != hipSuccess) {
         fail(err, err_len, "page-locked host memory for the rows and logits");
@@ -963,7 +970,8 @@ extern "C" bool vitna_cuda_moe_head(struct vitna_cuda_model* g, float* logits, c
     if (!g || g->lost) return fail(err, err_len, "the device model is not usable");
     if (!g->attention) return fail(err, err_len, "this model has no output projection");
     if (!check_launch(g, enqueue_head(g), "the head", err, err_len)) return false;
-    if (logits) HIP_TRY(hipMemcpyAsync(logits, g->vocab, (size_t)g->V * 4, hipMemcpyDeviceToHost, g->stream), "copying the logits");
+    void* const out[1] = {logits};
+    HIP_TRY(host_copy_rows(g->results, g->stream, g->vocab, (size_t)g->V * 4, 1, out), "copying the logits");
     HIP_TRY(hipStreamSynchronize(g->stream), "running the head");
     return true;
 }
@@ -1330,7 +1338,8 @@ extern "C" bool vitna_hip_moe_step(struct vitna_cuda_model* g, size_t seq, int32
                                    size_t err_len) {
     if (g && !experts_resident(g, err, err_len)) return false;
     if (!vitna_hip_moe_step_async(g, seq, token, pos, err, err_len)) return false;
-    if (logits) HIP_TRY(hipMemcpyAsync(logits, g->vocab, (size_t)g->V * 4, hipMemcpyDeviceToHost, g->stream), "copying the logits");
+    void* const out[1] = {logits};
+    HIP_TRY(host_copy_rows(g->results, g->stream, g->vocab, (size_t)g->V * 4, 1, out), "copying the logits");
     HIP_TRY(hipStreamSynchronize(g->stream), "running the step");
     return !g->last_step_mega || step_check(g, err, err_len);
 }
@@ -1739,23 +1748,27 @@ static bool prefill_check(vitna_cuda_model* g, size_t layer, size_t n, char* err
 
 extern "C" bool vitna_hip_moe_prefill(struct vitna_cuda_model* g, size_t layer, float* x, size_t n, int32_t* chosen, char* err,
                                       size_t err_len) {
+    return vitna_hip_moe_prefill_to(g, layer, x, n, x, chosen, err, err_len);
+}
+
+extern "C" bool vitna_hip_moe_prefill_to(struct vitna_cuda_model* g, size_t layer, const float* x, size_t n, float* out, int32_t* chosen,
+                                         char* err, size_t err_len) {
     if (g && !experts_resident(g, err, err_len)) return false;
     if (!prefill_check(g, layer, n, err, err_len)) return false;
-    if (!x) return fail(err, err_len, "no rows");
+    if (!x || !out) return fail(err, err_len, "no rows");
     HIP_TRY(hipSetDevice(g->device), "selecting the model's device");
     if (!prefill_reserve(g, n, err, err_len)) return false;
     HIP_TRY(hipMemcpyAsync(g->pf_x, x, n * g->H * 4, hipMemcpyHostToDevice, g->stream), "copying the rows to the device");
     if (!check_launch(g, enqueue_prefill(g, (int)layer, (int)n, g->pf_x, g->pf, nullptr), "the prefill", err, err_len)) return false;
-    HIP_TRY(hipMemcpyAsync(x, g->pf_x, n * g->H * 4, hipMemcpyDeviceToHost, g->stream), "copying the rows back");
-    if (chosen) {
-        std::vector<route_out> rt(n);
-        HIP_TRY(hipMemcpyAsync(rt.data(), g->pf.rt, n * sizeof(route_out), hipMemcpyDeviceToHost, g->stream), "copying the routing");
-        if (!sync_stream(g, "the prefill", err, err_len)) return false;
-        for (size_t i = 0; i < n; i++)
-            for (int k = 0; k < g->K; k++) chosen[i * g->K + k] = rt[i].chosen[k];
-        return true;
-    }
-    return sync_stream(g, "the prefill", err, err_len);
+    void* const rows[1] = {out};
+    HIP_TRY(host_copy_rows(g->results, g->stream, g->pf_x, n * g->H * 4, 1, rows), "copying the rows back");
+    if (!chosen) return true;
+    /* the experts' partial outputs are added up: their room takes the list of experts */
+    int32_t* list = reinterpret_cast<int32_t*>(g->pf.ypart);
+    if (!check_launch(g, launch_prefill_chosen(g->pf.rt, (int)n, g->K, list, g->stream), "the prefill", err, err_len)) return false;
+    void* const ids[1] = {chosen};
+    HIP_TRY(host_copy_rows(g->results, g->stream, list, n * g->K * 4, 1, ids), "copying the routing");
+    return true;
 }
 
 extern "C" bool vitna_hip_time_prefill(struct vitna_cuda_model* g, size_t layer, size_t n, uint64_t seed, int reps, double* us_total,
@@ -2359,12 +2372,14 @@ extern "C" bool vitna_hip_set_exact_rows(struct vitna_cuda_model* g, size_t n, c
 static bool set_rows(vitna_cuda_model* g, const vitna_cuda_row_t* rows, size_t n, char* err, size_t err_len) {
     if (n < 1 || n > ROWS_MAX) return fail(err, err_len, "%zu rows: 1 to %d a pass", n, ROWS_MAX);
     bool shared = false;
+    const uint64_t pass = ++g->seq_pass;
     for (size_t i = 0; i < n; i++) {
         const vitna_cuda_row_t r = rows[i];
         if (r.seq < 0 || r.seq >= g->seqs) return fail(err, err_len, "row %zu: sequence %d, the cache holds %d", i, r.seq, g->seqs);
         if (r.pos < 0 || r.pos >= g->ctx) return fail(err, err_len, "row %zu: position %d, the cache holds %d", i, r.pos, g->ctx);
         if (r.token < 0 || r.token >= g->V) return fail(err, err_len, "row %zu: token %d outside the vocabulary of %d", i, r.token, g->V);
-        for (size_t j = 0; j < i; j++) shared |= rows[j].seq == r.seq;
+        shared |= g->seq_seen[r.seq] == pass;
+        g->seq_seen[r.seq] = pass;
     }
     HIP_TRY(hipEventSynchronize(g->rows_copied), "waiting for the previous row copy");
     g->row_set = false;
@@ -2590,9 +2605,8 @@ extern "C" bool vitna_cuda_moe_rows_head(struct vitna_cuda_model* g, size_t n, f
     if (head == HEAD_NONE) return true;
     if (!check_launch(g, g->pass_exact ? enqueue_exact_head(g, (int)n) : enqueue_rows_head(g, (int)n, nullptr, head), "the head", err, err_len))
         return false;
-    for (size_t i = 0; i < n; i++)
-        if (logits && logits[i])
-            HIP_TRY(hipMemcpyAsync(logits[i], g->vocab + i * g->V, (size_t)g->V * 4, hipMemcpyDeviceToHost, g->stream), "copying logits");
+    if (logits)
+        HIP_TRY(host_copy_rows(g->results, g->stream, g->vocab, (size_t)g->V * 4, n, reinterpret_cast<void* const*>(logits)), "copying logits");
     HIP_TRY(hipStreamSynchronize(g->stream), "running the head");
     return true;
 }
@@ -2680,9 +2694,8 @@ extern "C" bool vitna_hip_moe_rows_step(struct vitna_cuda_model* g, const vitna_
     if (!ensure_rows_graph(g, (int)n, head_rows(g, n, logits), err, err_len)) return false;
     HIP_TRY(hipGraphLaunch(g->rg[g->rg_cur].exec, g->stream), "launching the rows step");
     g->last_step_mega = false;
-    for (size_t i = 0; i < n; i++)
-        if (logits && logits[i])
-            HIP_TRY(hipMemcpyAsync(logits[i], g->vocab + i * g->V, (size_t)g->V * 4, hipMemcpyDeviceToHost, g->stream), "copying logits");
+    if (logits)
+        HIP_TRY(host_copy_rows(g->results, g->stream, g->vocab, (size_t)g->V * 4, n, reinterpret_cast<void* const*>(logits)), "copying logits");
     if (logits) HIP_TRY(hipStreamSynchronize(g->stream), "running the rows step");
     return true;
 }
