@@ -37,11 +37,13 @@
 #define ROWS_MAX 1024
 /* passes of this many rows or more, of a model whose experts are resident, take the grouped kernels on tiles of
    32 pairs (launch_gsx) instead of four (launch_gmma_in / _down). At top-8 of 128 experts (a 4096-token prompt
-   in chunks, same box): 96-row chunks 961 -> 781 ms, 128 903 -> 707, 256 635 -> 433, 1024 415 -> 250; the
-   32 rows of a ragged step (two pairs an expert) 12.55 -> 17.74 ms, so they keep the four-pair tiles */
+   in chunks, same box): 96-row chunks 961 -> 781 ms, 128 903 -> 707, 256 635 -> 433, 1024 415 -> 250 with one
+   superblock of a tile a wave, and the kernels that loop over the width are 1.6 times as fast again; the 32 rows of
+   a ragged step (two pairs an expert) 12.55 -> 17.74 ms, so they keep the four-pair tiles */
 #define GSX_ROWS 64
-/* With the model's gpu_fast, a pass of at least this many rows runs its experts as the bf16 matrix-core grouped GEMM
-   of the prefill (the reference's FAST_ROWS, model_cuda.cu:204); smaller passes keep the exact kernels. */
+/* With the model's gpu_fast, a pass of at least this many rows runs its experts in 16-bit activations (K-quants on the
+   32-pair tiles, Q8_0 as the prefill's grouped GEMM; the reference's FAST_ROWS, model_cuda.cu:204); smaller passes
+   keep the exact kernels. */
 #define FAST_ROWS 64
 /* Passes of the rows ABI of at most exact_rows rows (model.c's PASS_MAX, 64: the passes that check drafted tokens
    and the batched steps of a server, model.c:1052-1190) run each row through the kernels of a single token's step,
