@@ -39,8 +39,9 @@
    32 pairs (launch_gsx) instead of four (launch_gmma_in / _down). At top-8 of 128 experts (a 4096-token prompt
    in chunks, same box): 96-row chunks 961 -> 781 ms, 128 903 -> 707, 256 635 -> 433, 1024 415 -> 250 with one
    superblock of a tile a wave, and the kernels that loop over the width are 1.6 times as fast again; the 32 rows of
-   a ragged step (two pairs an expert) 12.55 -> 17.74 ms, so they keep the four-pair tiles */
-#define GSX_ROWS 64
+   a ragged step (two pairs an expert) 12.55 -> 17.74 ms, so they keep the four-pair tiles. Not from 64: a 65-row
+   pass on a small ill-conditioned model came to 1.07e-3 of a step's logits on the 32-pair tiles (bound 1e-3) */
+#define GSX_ROWS 72
 /* With the model's gpu_fast, a pass of at least this many rows runs its experts in 16-bit activations (K-quants on the
    32-pair tiles, Q8_0 as the prefill's grouped GEMM; the reference's FAST_ROWS, model_cuda.cu:204); smaller passes
    keep the exact kernels. */
