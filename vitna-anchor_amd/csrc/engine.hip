@@ -132,7 +132,8 @@ struct vitna_cuda_model {
         hipGraph_t src;
         hipGraphExec_t exec;
         int n;                  /* rows, or 0 for an empty entry */
-        bool shared, fast;      /* rows of one sequence; the experts as the grouped GEMM */
+        bool shared, one_seq;   /* two rows or more of one sequence; all of them (attention over tiles of rows) */
+        bool fast;              /* the experts in 16-bit activations */
         int splits;             /* the attention's grid */
         int head;               /* the head's rows: HEAD_ALL, HEAD_NONE or the one row */
         uint64_t used;
@@ -2654,7 +2655,7 @@ static bool ensure_rows_graph(vitna_cuda_model* g, int n, int head, char* err, s
     int pick = 0;
     for (int i = 0; i < ROWS_GRAPHS; i++) {
         const auto& r = g->rg[i];
-        if (r.n == n && r.shared == g->rows_shared_seq && r.fast == fast && r.splits == g->splits_grid && r.head == head) {
+        if (r.n == n && r.shared == g->rows_shared_seq && r.one_seq == g->rows_one_seq && r.fast == fast && r.splits == g->splits_grid && r.head == head) {
             g->rg[i].used = ++g->rg_clock;
             g->rg_cur = i;
             return true;
@@ -2681,6 +2682,7 @@ static bool ensure_rows_graph(vitna_cuda_model* g, int n, int head, char* err, s
     r.n = n;
     r.fast = fast;
     r.shared = g->rows_shared_seq;
+    r.one_seq = g->rows_one_seq;
     r.splits = g->splits_grid;
     r.head = head;
     r.used = ++g->rg_clock;
