@@ -129,3 +129,48 @@ def test_fast_tile_edges(gate_up, down, hidden, inter):
     finally:
         dev.close()
         model.free()
+
+
+def given_rows(model, dev, n):
+    """A pass of n rows of one sequence up to its experts: their residual rows and normalized rows."""
+    cfg = model.cfg
+    dev.rows_route([((11 * i + 7) % cfg.vocab, i, 0) for i in range(n)], 0)
+    norm = np.ctypeslib.as_array(model.m.layers[0].mlp_norm, shape=(cfg.hidden,)).copy()
+    x0 = np.stack([dev.residual(i) for i in range(n)])
+    return x0, np.stack([oracle.rmsnorm(x, norm, cfg.rms_eps) for x in x0])
+
+
+def check_mixture(model, dev, n, K, seed, bar):
+    """The mixture of n given rows against the oracle's, to bar and what float32 keeps of it beside its residual row."""
+    x0, xn = given_rows(model, dev, n)
+    ids, w = routing(n, model.cfg.n_experts, K, seed)
+    dev.rows_experts(0, ids, w)
+    worst = 0.0
+    for i in range(n):
+        ref = mixture(model, 0, xn[i], ids[i], w[i]).astype(np.float64)
+        got = dev.residual(i).astype(np.float64) - x0[i]
+        assert np.isfinite(ref).all() and np.isfinite(got).all(), ("row", i)
+        most = float(np.max(np.abs(ref)))
+        lost = float(np.max(np.abs(x0[i].astype(np.float64) + ref))) * 2.0 ** -23 / most
+        r = float(np.max(np.abs(got - ref)) / most)
+        worst = max(worst, r)
+        assert r <= bar + lost, ("row", i, r, lost)
+    say("  worst rel err of the mixture", worst)
+
+
+@pytest.mark.parametrize("gate_up,down,scale", [(va.Q8_0, va.Q6_K, 2.0 ** 62), (va.Q4_K, va.Q8_0, 2.0 ** 59), (va.Q6_K, va.Q8_0, 2.0 ** 60)])
+def test_large_activations(gate_up, down, scale):
+    """Norm weights of 2^60: normalized rows of that size and SwiGLU outputs above 2^116, which the f16 operands hold by the
+    row's own power of two; the mixture is finite, as in float32."""
+    say("large activations", gate_up, down)
+    model = va.Model(va.shape(n_layers=1, hidden=256, intermediate=256, n_heads=4, n_kv_heads=2, head_dim=64, vocab=300, n_experts=24,
+                              n_experts_used=4, renormalize=0, dt_gate_up=gate_up, dt_down=down, norm_std=0.5, k_scale=1e-4,
+                              q8_scale=0.02 / 127, ctx=208, seqs=1), 980)
+    norm = np.ctypeslib.as_array(model.m.layers[0].mlp_norm, shape=(256,))
+    norm *= np.float32(scale)
+    dev = va.Device(model)
+    try:
+        check_mixture(model, dev, 200, 4, 7, REL)
+    finally:
+        dev.close()
+        model.free()

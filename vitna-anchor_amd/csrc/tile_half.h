@@ -39,12 +39,11 @@ __device__ __forceinline__ h2 th_h2(uint32_t v) { return __builtin_bit_cast(h2, 
 __device__ __forceinline__ h2 th_both(_Float16 v) { return h2{v, v}; }
 __device__ __forceinline__ h8 th_join(h2 a, h2 b, h2 c, h2 d) { return h8{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y}; }
 
-/* The power of two that brings a row's largest magnitude under 2^14 (1 for a row of zeros or one that is not
-   finite, whose results are not either way). */
+/* The power of two that brings a row's largest magnitude under 2^14 (1 for a row that is not finite, whose results are
+   not either way), its inverse a normal number too. */
 __device__ __forceinline__ float th_scale(float largest) {
     const int e = (int)(__float_as_uint(largest) >> 23) & 0xff;
-    if (e == 0 || e == 0xff) return 1.0f;
-    return __uint_as_float((uint32_t)(min(max(13 - (e - 127), -100), 100) + 127) << 23);
+    return e == 0xff ? 1.0f : __uint_as_float((uint32_t)(min(13 - (e - 127), 126) + 127) << 23);
 }
 
 /* eight values times f as f16 hi and lo in the operands' order, and the sum of hi + lo (fast: of hi) */
