@@ -174,3 +174,24 @@ def test_large_activations(gate_up, down, scale):
     finally:
         dev.close()
         model.free()
+
+
+def all_of(dtype):
+    return {"dt_" + m: dtype for m in ("q", "k", "v", "o", "embed")}
+
+
+@pytest.mark.parametrize("gate_up,down,k_scale,q8_scale,eps", [(va.Q8_0, va.Q6_K, 1e-4, 10000.0, 2.0 ** 48), (va.Q4_K, va.Q8_0, 10000.0, 1e-3, 2.0 ** 60),
+                                                               (va.Q6_K, va.Q8_0, 3000.0, 1e-3, 2.0 ** 54)])
+def test_rows_far_below_their_bound(gate_up, down, k_scale, q8_scale, eps):
+    """An epsilon that makes normalized rows some 2^-30 of the largest that the norm's weights allow: a row's operands hold
+    it as well as any other's, so its mixture is within the same bar."""
+    say("rows far below their bound", gate_up, down)
+    model = va.Model(va.shape(n_layers=1, hidden=256, intermediate=256, n_heads=4, n_kv_heads=2, head_dim=64, vocab=300, n_experts=24,
+                              n_experts_used=4, renormalize=0, dt_gate_up=gate_up, dt_down=down, norm_std=0.5, k_scale=k_scale,
+                              q8_scale=q8_scale, rms_eps=eps, ctx=208, seqs=1, **all_of(va.Q4_K if gate_up == va.Q8_0 else va.Q8_0)), 980)
+    dev = va.Device(model)
+    try:
+        check_mixture(model, dev, 200, 4, 8, REL)
+    finally:
+        dev.close()
+        model.free()

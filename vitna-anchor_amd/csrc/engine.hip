@@ -28,7 +28,6 @@
 #include <string.h>
 #include <vector>
 #include <algorithm>
-#include <cmath>
 #include <type_traits>
 #include <mutex>
 
@@ -60,7 +59,6 @@
 struct dlayer {
     qmat q, k, v, o;
     float *attn_norm, *mlp_norm, *q_norm, *k_norm;
-    float mlp_scale; /* norm_scale of mlp_norm */
     float* router;
     qmat gate, up, down;
     /* the experts' copies tiled for the crowded passes' grouped kernels (launch_gsx), or null */
@@ -122,7 +120,7 @@ struct vitna_cuda_model {
     int *gsx_toff, *gsx_te, *gsx_tb;
     uint32_t *gsx_img_in, *gsx_img_act;
     uint16_t* gsx_sums;
-    float *gsx_act, *gsx_inv;
+    float *gsx_act, *gsx_scale, *gsx_inv;
     std::vector<uint64_t> seq_seen; /* by sequence: the last pass (seq_pass) that had a row of it */
     uint64_t seq_pass;
     bool rows_shared_seq;       /* the pass's rows include two of one sequence (attention prepares first) */
@@ -367,16 +365,6 @@ static bool upload_set(vitna_cuda_model* g, const vitna_matrix_t* const* mats, s
     return true;
 }
 
-/* The power of two that brings every value of a row normalized with weights w under 2^14 (a normalized row's values
-   are at most sqrt(n) before the weights); 1 where the weights are zero or not finite. */
-static float norm_scale(const float* w, size_t n) {
-    double largest = 0.0;
-    for (size_t i = 0; i < n; i++) largest = std::max(largest, std::fabs((double)w[i]));
-    const double bound = largest * std::sqrt((double)n) * 1.0001;
-    if (!(bound > 0.0) || !std::isfinite(bound)) return 1.0f;
-    return (float)std::ldexp(1.0, std::min(std::max(13 - std::ilogb(bound), -100), 100));
-}
-
 static bool upload_f32(vitna_cuda_model* g, float** out, const float* host, size_t n, const char* what, char* err, size_t err_len) {
     if (!dalloc(g, out, n * 4, what, err, err_len)) return false;
     HIP_TRY(hipMemcpy(*out, host, n * 4, hipMemcpyHostToDevice), what);
@@ -431,7 +419,7 @@ static bool ensure_tiled(vitna_cuda_model* g, char* err, size_t err_len) {
        spare): without it those passes keep the four-pair kernels */
     if (!g->ec.on && g->E <= ROUTE_E_MAX && gsx_fits(g->L[0].gate, g->L[0].up, g->L[0].down)) {
         const size_t T = (size_t)gsx_max_tiles(ROWS_MAX, g->K, g->E), H = g->H, I = g->L[0].gate.rows, W = std::max(H, I);
-        size_t need = (g->E + 2 + 2 * T) * sizeof(int) + 32 * T * (H + 2 * I) * 4 + T * (W / 256) * 1024 + 32 * T * 4;
+        size_t need = (g->E + 2 + 2 * T) * sizeof(int) + 32 * T * (H + 2 * I) * 4 + T * (W / 256) * 1024 + (ROWS_MAX + 32 * T) * 4;
         for (int l = 0; l < g->NL; l++) {
             const dlayer& d = g->L[l];
             if (gsx_fits(d.gate, d.up, d.down))
@@ -445,6 +433,7 @@ static bool ensure_tiled(vitna_cuda_model* g, char* err, size_t err_len) {
                   dalloc(g, &g->gsx_img_in, 32 * T * H * 4, "scratch", err, err_len) &&
                   dalloc(g, &g->gsx_img_act, 32 * T * I * 4, "scratch", err, err_len) &&
                   dalloc(g, &g->gsx_sums, T * (W / 256) * 1024, "scratch", err, err_len) &&
+                  dalloc(g, &g->gsx_scale, ROWS_MAX * 4, "scratch", err, err_len) &&
                   dalloc(g, &g->gsx_inv, 32 * T * 4, "scratch", err, err_len) &&
                   dalloc(g, &g->gsx_act, 32 * T * I * 4, "scratch", err, err_len)))
                 return false;
@@ -584,7 +573,6 @@ extern "C" struct vitna_cuda_model* vitna_cuda_create(const vitna_llama_t* m, co
         const vitna_llama_layer_t* L = &m->layers[l];
         dlayer& d = g->L[l];
         memset(&d, 0, sizeof(d));
-        d.mlp_scale = norm_scale(L->mlp_norm, c->hidden);
         ok = upload_f32(g, &d.mlp_norm, L->mlp_norm, c->hidden, "the MLP norm", err, err_len) &&
              upload_f32(g, &d.router, (const float*)L->router.data, c->n_experts * c->hidden, "the router", err, err_len);
         const vitna_expert_t* x0 = &L->experts[0];
@@ -2220,7 +2208,7 @@ static hipError_t enqueue_rows_experts(vitna_cuda_model* g, int layer, int n, bo
         x.xn = g->xn; x.rt = rt; x.count = g->grp_count; x.pairs = g->grp_pairs;
         x.E = g->E; x.K = g->K; x.cap = ROWS_MAX; x.n = n; x.fast = rows_fast(g, n);
         x.toff = g->gsx_toff; x.te = g->gsx_te; x.tb = g->gsx_tb; x.max_tiles = gsx_max_tiles(ROWS_MAX, g->K, g->E);
-        x.img_in = g->gsx_img_in; x.img_act = g->gsx_img_act; x.sums = g->gsx_sums; x.xscale = d.mlp_scale; x.inv = g->gsx_inv;
+        x.img_in = g->gsx_img_in; x.img_act = g->gsx_img_act; x.sums = g->gsx_sums; x.scale = g->gsx_scale; x.inv = g->gsx_inv;
         x.act = g->gsx_act; x.ypart = g->ypart;
         e = launch_gsx(x, g->stream);
         if (e == hipSuccess && !defer_sum) e = launch_reduce_rows(g->ypart, g->x, n, g->K, g->H, g->stream);

@@ -409,14 +409,32 @@ bool gsx_fits(const qmat& gate, const qmat& up, const qmat& down) {
 int gsx_max_tiles(int n, int K, int E) { return (n * K + 31) / 32 + E; }
 int gsx_max_blocks(int n, int K, int E) { return (n * K + 63) / 64 + E; }
 
+__device__ __forceinline__ float gsx_largest(float m, const float4& v) {
+    return fmaxf(m, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+}
+
 /* Tile offsets of the experts' pair lists (toff[E + 1]), the expert of each tile (te[max_tiles], -1 past the
-   last) and the first tile of each token block of up to `block` tiles (tb, their number at n_tb): one block, the first wave scanning the
-   tile counts, the second the block counts, 64 experts at a time. */
+   last) and the first tile of each token block of up to `block` tiles (tb, their number at n_tb): block 0, the first
+   wave scanning the tile counts, the second the block counts, 64 experts at a time. The blocks after it take four
+   rows each of the n (H wide) at x and leave the rows' powers of two in scale: beside the plan, which one block
+   takes longer over. */
 __global__ __launch_bounds__(256) void gsx_plan_kernel(const int* __restrict__ count, int E, int* __restrict__ toff,
                                                        int* __restrict__ te, int max_tiles, int block, int* __restrict__ tb,
-                                                       int* __restrict__ n_tb) {
+                                                       int* __restrict__ n_tb, const float* __restrict__ x, int n, int H,
+                                                       float* __restrict__ scale) {
     __shared__ int off[2][ROUTE_E_MAX + 1];
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    if (blockIdx.x) {
+        const int row = 4 * (blockIdx.x - 1) + wv;
+        if (row >= n) return;
+        const float4* src = reinterpret_cast<const float4*>(x + (size_t)row * H);
+        float m = 0.0f;
+        for (int c = lane; c < H / 4; c += 64) m = gsx_largest(m, src[c]);
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) m = fmaxf(m, __shfl_xor(m, d, WAVE));
+        if (lane == 0) scale[row] = th_scale(m);
+        return;
+    }
     if (wv < 2) {
         const int per = wv ? 32 * block : 32;
         int run = 0;
@@ -461,7 +479,7 @@ __device__ __forceinline__ int gsx_tiles(const int* __restrict__ te, int t, int 
 template <int DT, bool FAST>
 __global__ __launch_bounds__(TG_THREADS) void gsx_tile_in_kernel(qmat gate, qmat up, tg_images im, const int* __restrict__ te,
                                                                  const int* __restrict__ tb, const int* __restrict__ n_tb, int T,
-                                                                 float inv, float* __restrict__ act) {
+                                                                 const float* __restrict__ inv, float* __restrict__ act) {
     __shared__ __attribute__((aligned(1024))) uint8_t lds[tg_lds<DT>::BYTES];
     constexpr int NT = FAST ? 2 : 1;
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -484,8 +502,9 @@ __global__ __launch_bounds__(TG_THREADS) void gsx_tile_in_kernel(qmat gate, qmat
 #pragma unroll
         for (int r = 0; r < 16; r++) {
             const int tok = 8 * (r >> 2) + 4 * kq + (r & 3);
-            const float g = acc[j][0][r] * inv;
-            act[(size_t)(32 * (t + NT * tg + j) + tok) * I + 32 * (4 * x + rg) + l32] = (g / (1.0f + expf(-g))) * (acc[j][1][r] * inv);
+            const size_t row = 32 * (t + NT * tg + j) + tok;
+            const float f = inv[row], g = acc[j][0][r] * f;
+            act[row * I + 32 * (4 * x + rg) + l32] = (g / (1.0f + expf(-g))) * (acc[j][1][r] * f);
         }
     }
 }
@@ -546,11 +565,12 @@ __device__ __forceinline__ void gsx_put(u32x4* img, bool order_b, bool fast, int
 
 /* The images (one column order) and, for Q4_K weights, group sums of the virtual token tiles: block (b, t) takes
    superblock b of tile t, whose token l is pair 32 (t - toff[e]) + l of expert te[t] (past its count: the last pair
-   again), row pair / ROUTE_K_MAX of x, times f (every row's values stay under 2^14). */
-__global__ __launch_bounds__(256) void gsx_image_kernel(const float* __restrict__ x, int K, float f, const int* __restrict__ pairs,
-                                                        const int* __restrict__ count, int cap, const int* __restrict__ toff,
-                                                        const int* __restrict__ te, u32x4* __restrict__ img, bool order_b, bool fast,
-                                                        _Float16* __restrict__ sums) {
+   again), row pair / ROUTE_K_MAX of x, times that row's scale, whose inverse goes to inv. */
+__global__ __launch_bounds__(256) void gsx_image_kernel(const float* __restrict__ x, int K, const float* __restrict__ scale,
+                                                        const int* __restrict__ pairs, const int* __restrict__ count, int cap,
+                                                        const int* __restrict__ toff, const int* __restrict__ te,
+                                                        u32x4* __restrict__ img, bool order_b, bool fast, _Float16* __restrict__ sums,
+                                                        float* __restrict__ inv) {
     const int b = blockIdx.x, t = blockIdx.y;
     const int e = te[t];
     if (e < 0) return;
@@ -562,6 +582,8 @@ __global__ __launch_bounds__(256) void gsx_image_kernel(const float* __restrict_
         const float4* src = reinterpret_cast<const float4*>(x + src_row * K + 8 * c8);
         const float4 v0 = src[0], v1 = src[1];
         const float ev[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
+        const float f = scale[src_row];
+        if (c8 == 0) inv[32 * t + l] = 1.0f / f;
         u32x4 vh, vl;
         float sum;
         th_split8(ev, f, fast, vh, vl, sum);
@@ -582,9 +604,7 @@ __global__ __launch_bounds__(256) void gsx_act_image_kernel(const float* __restr
     const float4* src = reinterpret_cast<const float4*>(x + (size_t)row * K);
     float m = 0.0f;
     for (int c = j; c < K / 8; c += 8) {
-        const float4 v0 = src[2 * c], v1 = src[2 * c + 1];
-        const float a = fmaxf(fmaxf(fabsf(v0.x), fabsf(v0.y)), fmaxf(fabsf(v0.z), fabsf(v0.w)));
-        m = fmaxf(m, fmaxf(a, fmaxf(fmaxf(fabsf(v1.x), fabsf(v1.y)), fmaxf(fabsf(v1.z), fabsf(v1.w)))));
+        m = gsx_largest(gsx_largest(m, src[2 * c]), src[2 * c + 1]);
     }
 #pragma unroll
     for (int d = 1; d < 8; d <<= 1) m = fmaxf(m, __shfl_xor(m, d, WAVE));
@@ -612,7 +632,7 @@ static hipError_t launch_gsx_tiles(const gsx_args& a, bool in, hipStream_t s) {
     const int *tb = a.tb, *n_tb = a.tb + a.max_tiles;
     auto go = [&](auto dt) {
         constexpr int DT = decltype(dt)::value;
-        if (in) gsx_tile_in_kernel<DT, FAST><<<blocks, TG_THREADS, 0, s>>>(a.gate, a.up, k, a.te, tb, n_tb, T, 1.0f / a.xscale, a.act);
+        if (in) gsx_tile_in_kernel<DT, FAST><<<blocks, TG_THREADS, 0, s>>>(a.gate, a.up, k, a.te, tb, n_tb, T, a.inv, a.act);
         else gsx_tile_down_kernel<DT, FAST><<<blocks, TG_THREADS, 0, s>>>(a.down, k, a.te, tb, n_tb, T, a.toff, a.count, a.pairs, a.cap, a.rt, a.K, a.inv, a.ypart);
     };
     switch (m.dtype) {
@@ -626,18 +646,18 @@ static hipError_t launch_gsx_tiles(const gsx_args& a, bool in, hipStream_t s) {
     return hipGetLastError();
 }
 
-/* A row of normalized values is under sqrt(H) times the norm's largest weight; a.xscale keeps that under 2^14. */
 hipError_t launch_gsx(const gsx_args& a, hipStream_t s) {
     if (!gsx_fits(a.gate, a.up, a.down) || !a.gate.tiled || !a.up.tiled || !a.down.tiled || a.K < 1 || a.K > ROUTE_K_MAX ||
-        a.E < 1 || a.E > ROUTE_E_MAX || a.n < 1 || a.cap < a.n || a.max_tiles < gsx_max_tiles(a.n, a.K, a.E) || !(a.xscale > 0.0f))
+        a.E < 1 || a.E > ROUTE_E_MAX || a.n < 1 || a.cap < a.n || a.max_tiles < gsx_max_tiles(a.n, a.K, a.E))
         return hipErrorInvalidValue;
     const int H = a.gate.cols, I = a.gate.rows, T = gsx_max_tiles(a.n, a.K, a.E);
-    gsx_plan_kernel<<<1, 256, 0, s>>>(a.count, a.E, a.toff, a.te, T, a.fast ? 4 : 2, a.tb, a.tb + a.max_tiles);
+    gsx_plan_kernel<<<1 + (a.n + 3) / 4, 256, 0, s>>>(a.count, a.E, a.toff, a.te, T, a.fast ? 4 : 2, a.tb, a.tb + a.max_tiles, a.xn, a.n, H,
+                                                      a.scale);
     u32x4* ii = reinterpret_cast<u32x4*>(a.img_in);
     u32x4* ia = reinterpret_cast<u32x4*>(a.img_act);
     _Float16* sums = reinterpret_cast<_Float16*>(a.sums);
-    gsx_image_kernel<<<dim3(H / 256, T), 256, 0, s>>>(a.xn, H, a.xscale, a.pairs, a.count, a.cap, a.toff, a.te, ii,
-                                                      a.gate.dtype == VITNA_DTYPE_Q6_K, a.fast, sums);
+    gsx_image_kernel<<<dim3(H / 256, T), 256, 0, s>>>(a.xn, H, a.scale, a.pairs, a.count, a.cap, a.toff, a.te, ii,
+                                                      a.gate.dtype == VITNA_DTYPE_Q6_K, a.fast, sums, a.inv);
     hipError_t err = a.fast ? launch_gsx_tiles<true>(a, true, s) : launch_gsx_tiles<false>(a, true, s);
     if (err != hipSuccess) return err;
     gsx_act_image_kernel<<<T, 256, 0, s>>>(a.act, I, a.te, ia, a.down.dtype == VITNA_DTYPE_Q6_K, a.fast, sums, a.inv);

@@ -331,8 +331,8 @@ struct gsx_args {
     uint32_t* img_in;      /* operand images of the tiles' rows: 32 max_tiles x H x 4 bytes */
     uint32_t* img_act;     /* of the SwiGLU output: 32 max_tiles x I x 4 bytes */
     uint16_t* sums;        /* group sums: max_tiles x (max(H, I) / 256) x 1024 bytes */
-    float xscale;          /* the power of two that keeps xn's values under 2^14 */
-    float* inv;            /* [32 max_tiles]: the inverse of each SwiGLU row's power of two */
+    float* scale;          /* [cap]: the power of two that brings each row of xn into f16 */
+    float* inv;            /* [32 max_tiles]: the inverse of each operand row's power of two, xn's and then the SwiGLU output's */
     float* act;            /* the SwiGLU output [32 max_tiles][I] */
     float* ypart;          /* [n][K][H] */
 };
