@@ -419,7 +419,7 @@ static bool ensure_tiled(vitna_cuda_model* g, char* err, size_t err_len) {
        spare): without it those passes keep the four-pair kernels */
     if (!g->ec.on && g->E <= ROUTE_E_MAX && gsx_fits(g->L[0].gate, g->L[0].up, g->L[0].down)) {
         const size_t T = (size_t)gsx_max_tiles(ROWS_MAX, g->K, g->E), H = g->H, I = g->L[0].gate.rows, W = std::max(H, I);
-        size_t need = (g->E + 2 + 2 * T) * sizeof(int) + 32 * T * (H + 2 * I) * 4 + T * (W / 256) * 1024 + (ROWS_MAX + 32 * T) * 4;
+        size_t need = (g->E + 2 + 2 * T) * sizeof(int) + 32 * T * (H + 2 * I) * 4 + T * (W / 256) * 2048 + (ROWS_MAX + 32 * T) * 4;
         for (int l = 0; l < g->NL; l++) {
             const dlayer& d = g->L[l];
             if (gsx_fits(d.gate, d.up, d.down))
@@ -432,7 +432,7 @@ static bool ensure_tiled(vitna_cuda_model* g, char* err, size_t err_len) {
                   dalloc(g, &g->gsx_tb, (T + 1) * sizeof(int), "scratch", err, err_len) &&
                   dalloc(g, &g->gsx_img_in, 32 * T * H * 4, "scratch", err, err_len) &&
                   dalloc(g, &g->gsx_img_act, 32 * T * I * 4, "scratch", err, err_len) &&
-                  dalloc(g, &g->gsx_sums, T * (W / 256) * 1024, "scratch", err, err_len) &&
+                  dalloc(g, &g->gsx_sums, T * (W / 256) * 2048, "scratch", err, err_len) &&
                   dalloc(g, &g->gsx_scale, ROWS_MAX * 4, "scratch", err, err_len) &&
                   dalloc(g, &g->gsx_inv, 32 * T * 4, "scratch", err, err_len) &&
                   dalloc(g, &g->gsx_act, 32 * T * I * 4, "scratch", err, err_len)))

@@ -59,7 +59,7 @@ template <int DT> struct tg_lds;
 template <> struct tg_lds<VITNA_DTYPE_Q4_K> {
     static constexpr int TB = 4608, WU = 1024, HDR_LANES = 32;
     static constexpr int HDR = 4 * (TG_T * 8192 + TG_R * WU); /* [8][512] */
-    static constexpr int SUMS = HDR + TG_R * 512;             /* [2][1024], FAST [4][1024] */
+    static constexpr int SUMS = HDR + TG_R * 512;             /* [2 tiles][2 pieces][1024], FAST [4 tiles][1024] */
     static constexpr int BYTES = SUMS + 2 * TG_T * 1024;
     static constexpr int loads(int u) { return TG_T + 1 + (u == 0); }
 };
@@ -116,7 +116,7 @@ __device__ __forceinline__ void tg_part(const tg_src& s, int b, uint32_t lds, in
             tg_dma(w + 4096 + (U / 2) * 1024, off, lds + L::QH + ((U / 2) * TG_R + wv) * 1024);
         if constexpr (U == 0) {
             if (lane < L::HDR_LANES) tg_dma(w + 4 * L::WU + (DT == VITNA_DTYPE_Q6_K ? 2048 : 0), off, lds + L::HDR + wv * L::HDR_LANES * 16);
-            if (DT == VITNA_DTYPE_Q4_K && wv < (FAST ? 2 : 1) * TG_T) tg_dma(s.sums + (size_t)b * 1024, off, lds + L::SUMS + wv * 1024);
+            if (DT == VITNA_DTYPE_Q4_K && wv < 2 * TG_T) tg_dma(s.sums + (size_t)b * 2048, off, lds + L::SUMS + wv * 1024);
         }
     }
 }
@@ -228,15 +228,15 @@ __device__ __forceinline__ void tg_body(const tg_src& s, int S, const uint8_t* l
     tg_a x[2];       /* the activations of this step and the next, by the step's parity */
     th_b<DT> o[2];   /* the weights of this step */
     h8 mins[2];      /* Q4_K: a superblock's minimums */
-    u32x4 sums[NT];  /* and its sums */
+    u32x4 sums[2];   /* and its sums: the token tile's two pieces, FAST its two tiles' */
     f32x16 P[NT][2] = {}, M[2]; /* the products, with their scale dP once they are finished, and Q4_K's of the minimums */
     float dP[2] = {0.0f, 0.0f}, dM[2] = {0.0f, 0.0f};
     auto start = [&](const sx_w<DT>(&ws)[2]) { /* a superblock's minimums and sums */
         if constexpr (Q4) {
 #pragma unroll
-            for (int t = 0; t < NT; t++) sums[t] = *(reinterpret_cast<const u32x4*>(lds + L::SUMS + (NT * tg + t) * 1024) + lane);
-            mins[0] = th_mins(th_header(ws[0]));
-            mins[1] = th_mins(th_header(ws[1]));
+            for (int t = 0; t < 2; t++) sums[t] = *(reinterpret_cast<const u32x4*>(lds + L::SUMS + (2 * tg + t) * 1024) + lane);
+            mins[0] = th_mins(th_header(ws[0]), lane >> 5);
+            mins[1] = th_mins(th_header(ws[1]), lane >> 5);
         }
     };
 #pragma unroll
@@ -253,8 +253,10 @@ __device__ __forceinline__ void tg_body(const tg_src& s, int S, const uint8_t* l
         auto step = [&](auto u, auto half) {
             constexpr int U = decltype(u)::value, N = decltype(half)::value, V = (U + 1) & 3;
             constexpr bool first = U == 0 && N == 0, last = U == 3 && N == 1;
-            /* a token tile's products of the minimums in one of the first steps, their scale in the next */
-            constexpr int mt = Q4 && 2 * U + N < NT ? 2 * U + N : -1, ms = Q4 && 2 * U + N >= 1 && 2 * U + N <= NT ? 2 * U + N - 1 : -1;
+            /* the minimums' products in the first two steps: FAST a token tile's in each, its scale in the next; else the
+               small piece's, then the large one's, and the scale in the third */
+            constexpr int mt = Q4 && 2 * U + N < 2 ? 2 * U + N : -1;
+            constexpr int ms = !Q4 ? -1 : FAST && (2 * U + N == 1 || 2 * U + N == 2) ? 2 * U + N - 1 : !FAST && 2 * U + N == 2 ? 0 : -1;
             __builtin_amdgcn_sched_barrier(0);
             sx_w<DT>(&ws)[2] = U == 3 ? wn : w; /* the next unit's */
             if constexpr (N == 0) {
@@ -286,7 +288,7 @@ __device__ __forceinline__ void tg_body(const tg_src& s, int S, const uint8_t* l
             if constexpr (mt >= 0) {
 #pragma unroll
                 for (int i = 0; i < 2; i++) {
-                    M[i] = TH_MMA(sums[mt], mins[i], f32x16{});
+                    M[i] = TH_MMA(sums[FAST ? mt : 1 - mt], mins[i], !FAST && mt == 1 ? M[i] : f32x16{});
                     if (mt == 0) dM[i] = th_dmin(w[i]);
                 }
             }
@@ -357,7 +359,7 @@ __device__ __forceinline__ void tg_body(const tg_src& s, int S, const uint8_t* l
 }
 
 /* What the kernels read: the rows' operand images (img, tile_half.h's values in skinny_image.h's layout, order B for
-   Q6_K; FAST: the hi pieces alone) and, for Q4_K, group sums ([tile][superblock][64][8] f16). */
+   Q6_K; FAST: the hi pieces alone) and, for Q4_K, group sums ([tile][superblock][2][64][8] f16, th_sum). */
 struct tg_images {
     const uint8_t *img, *sums;
 };
@@ -370,7 +372,7 @@ __device__ __forceinline__ tg_src tg_sources(const tg_images& a, const int (&tt)
     for (int j = 0; j < TG_T; j++)
         s.img[j] = FAST ? a.img + (size_t)tt[2 * j + (wv & 1)] * S * 16384 + (wv >> 1) * 1024 : a.img + (size_t)tt[j] * S * 32768 + wv * 1024;
     s.wt = tile;
-    s.sums = a.sums + (size_t)tt[wv & (FAST ? 3 : 1)] * S * 1024;
+    s.sums = FAST ? a.sums + (size_t)tt[wv & 3] * S * 2048 : a.sums + (size_t)tt[(wv >> 1) & 1] * S * 2048 + (wv & 1) * 1024;
     return s;
 }
 
@@ -590,7 +592,7 @@ __global__ __launch_bounds__(256) void gsx_image_kernel(const float* __restrict_
         gsx_put(img, order_b, fast, 32 * t + l, K, c8, vh, vl);
         if (order_b) continue;
         const float t16 = sum + __shfl_xor(sum, 1, WAVE), t32 = t16 + __shfl_xor(t16, 2, WAVE);
-        if (!(c8 & 3)) th_sum(sums + ((size_t)t * (K / 256) + b) * 512, l, (c8 & 31) >> 2, t32);
+        if (!(c8 & 3)) th_sum(sums + ((size_t)t * (K / 256) + b) * 1024, l, (c8 & 31) >> 2, t32);
     }
 }
 
@@ -619,7 +621,7 @@ __global__ __launch_bounds__(256) void gsx_act_image_kernel(const float* __restr
         gsx_put(img, order_b, fast, row, K, c, vh, vl);
         if (order_b) continue;
         const float t16 = sum + __shfl_xor(sum, 1, WAVE), t32 = t16 + __shfl_xor(t16, 2, WAVE);
-        if (!(c & 3)) th_sum(sums + ((size_t)t * (K / 256) + (c >> 5)) * 512, l, (c & 31) >> 2, t32);
+        if (!(c & 3)) th_sum(sums + ((size_t)t * (K / 256) + (c >> 5)) * 1024, l, (c & 31) >> 2, t32);
     }
 }
 

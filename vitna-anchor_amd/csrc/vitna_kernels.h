@@ -330,7 +330,7 @@ struct gsx_args {
     int max_tiles;         /* at least gsx_max_tiles(n, K, E) */
     uint32_t* img_in;      /* operand images of the tiles' rows: 32 max_tiles x H x 4 bytes */
     uint32_t* img_act;     /* of the SwiGLU output: 32 max_tiles x I x 4 bytes */
-    uint16_t* sums;        /* group sums: max_tiles x (max(H, I) / 256) x 1024 bytes */
+    uint16_t* sums;        /* group sums: max_tiles x (max(H, I) / 256) x 2048 bytes */
     float* scale;          /* [cap]: the power of two that brings each row of xn into f16 */
     float* inv;            /* [32 max_tiles]: the inverse of each operand row's power of two, xn's and then the SwiGLU output's */
     float* act;            /* the SwiGLU output [32 max_tiles][I] */
