@@ -140,10 +140,10 @@ def given_rows(model, dev, n):
     return x0, np.stack([oracle.rmsnorm(x, norm, cfg.rms_eps) for x in x0])
 
 
-def check_mixture(model, dev, n, K, seed, bar):
-    """The mixture of n given rows against the oracle's, to bar and what float32 keeps of it beside its residual row."""
+def check_mixture(model, dev, ids, w, bar):
+    """The mixture of given rows against the oracle's, to bar and what float32 keeps of it beside its residual row."""
+    n = len(ids)
     x0, xn = given_rows(model, dev, n)
-    ids, w = routing(n, model.cfg.n_experts, K, seed)
     dev.rows_experts(0, ids, w)
     worst = 0.0
     for i in range(n):
@@ -170,7 +170,7 @@ def test_large_activations(gate_up, down, scale):
     norm *= np.float32(scale)
     dev = va.Device(model)
     try:
-        check_mixture(model, dev, 200, 4, 7, REL)
+        check_mixture(model, dev, *routing(200, 24, 4, 7), REL)
     finally:
         dev.close()
         model.free()
@@ -191,7 +191,27 @@ def test_rows_far_below_their_bound(gate_up, down, k_scale, q8_scale, eps):
                               q8_scale=q8_scale, rms_eps=eps, ctx=208, seqs=1, **all_of(va.Q4_K if gate_up == va.Q8_0 else va.Q8_0)), 980)
     dev = va.Device(model)
     try:
-        check_mixture(model, dev, 200, 4, 8, REL)
+        check_mixture(model, dev, *routing(200, 24, 4, 8), REL)
+    finally:
+        dev.close()
+        model.free()
+
+
+@pytest.mark.parametrize("experts,gate_up,down", [(16, va.Q4_K, va.Q6_K), (16, va.Q6_K, va.Q4_K), (16, va.Q8_0, va.Q8_0), (40, va.Q4_K, va.Q6_K),
+                                                  (40, va.Q8_0, va.Q4_K)])
+@pytest.mark.parametrize("n", [63, 64, 71, 72, 95, 96])
+def test_first_tiled_passes(experts, gate_up, down, n):
+    """Passes about the first ones on the tiles: 64 rows, and 96 for K-quant experts with few blocks (16 experts of 512 x 256
+    have 32, 40 have 80), the kernels on either side of the limit to the grouped experts' bar."""
+    say("first tiled passes", experts, gate_up, down, n)
+    model = va.Model(va.shape(n_layers=1, hidden=512, intermediate=256, n_heads=4, n_kv_heads=2, head_dim=64, vocab=300, n_experts=experts,
+                              n_experts_used=4, renormalize=0, dt_gate_up=gate_up, dt_down=down, norm_std=0.5, ctx=n, seqs=1), 981)
+    dev = va.Device(model)
+    try:
+        dev.set_exact_rows(0)
+        rng = np.random.RandomState(n)
+        ids = np.stack([np.sort(rng.choice(experts, 4, replace=False)) for _ in range(n)]).astype(np.int32)
+        check_mixture(model, dev, ids, rng.uniform(0.05, 1.0, (n, 4)).astype(np.float32), REL)
     finally:
         dev.close()
         model.free()

@@ -34,13 +34,21 @@
 /* The most rows a pass takes (the reference's MOE_ROWS, model_cuda.cu:197): model.c runs a prompt in chunks of
    this many. Scratch for this many rows is allocated with the model. */
 #define ROWS_MAX 1024
-/* passes of this many rows or more, of a model whose experts are resident, take the grouped kernels on tiles of
-   32 pairs (launch_gsx) instead of four (launch_gmma_in / _down). At top-8 of 128 experts (a 4096-token prompt
-   in chunks, same box): 96-row chunks 961 -> 781 ms, 128 903 -> 707, 256 635 -> 433, 1024 415 -> 250 with one
-   superblock of a tile a wave, and the kernels that loop over the width are 1.6 times as fast again; the 32 rows of
-   a ragged step (two pairs an expert) 12.55 -> 17.74 ms, so they keep the four-pair tiles. Not from 64: a 65-row
-   pass on a small ill-conditioned model came to 1.07e-3 of a step's logits on the 32-pair tiles (bound 1e-3) */
-#define GSX_ROWS 72
+/* Passes of this many rows or more, of a model whose experts are resident, take the grouped kernels on tiles of
+   32 pairs (launch_gsx) instead of four (launch_gmma_in / _down). A rows step of four layers, top-8 of 128 experts of
+   2048 x 768, on the four-pair kernels and on the tiles, us: Q4_K_M 64 rows 945 and 795, 71 952 and 855, 96 1116 and
+   885, 128 1473 and 1068; Q8_0 64 rows 1361 and 805, 71 1387 and 861. The 32 rows of a ragged step (two pairs an
+   expert) 12.55 and 17.74 ms, and passes of 64 rows or fewer are mostly a step's kernels a row (EXACT_ROWS). */
+#define GSX_ROWS 64
+/* Of K-quant experts whose tile kernels would have GSX_FEW_BLOCKS blocks or fewer, a quarter of the compute units, it is
+   this many: each of those blocks walks the whole width alone, where the four-pair kernels spread an expert over more
+   of the chip. Rows steps of two layers, Q4_K_M, four-pair and tiles, us: 32 experts of 512 x 256 (64 blocks) 64 rows
+   170 and 189, 80 187 and 201, 96 195 and 205, 112 220 and 225, 128 257 and 254; 8 of 2048 x 2048 (64 blocks) 64 rows
+   264 and 351, 96 323 and 366, 160 482 and 461; in Q6_K they meet at 96 to 112 rows. With 128 blocks (32 of 1024 x
+   512) 64 rows 223 and 230, 80 249 and 240; Q8_0's four-pair kernels widen more and meet the tiles at 64 rows there
+   (16 experts of 1024 x 512: 229 and 225). */
+#define GSX_FEW_ROWS 96
+#define GSX_FEW_BLOCKS 64
 /* With the model's gpu_fast, a pass of at least this many rows runs its experts in 16-bit activations (K-quants on the
    32-pair tiles, Q8_0 as the prefill's grouped GEMM; the reference's FAST_ROWS, model_cuda.cu:204); smaller passes
    keep the exact kernels. */
@@ -2158,7 +2166,9 @@ static bool rows_fast(const vitna_cuda_model* g, int n) { return g->fast && (siz
 static bool rows_tiled(const vitna_cuda_model* g, int layer, int n) {
     const dlayer& d = g->L[layer];
     if (n < GSX_ROWS || !d.sx_gate) return false;
-    return !rows_fast(g, n) || (d.gate.dtype != VITNA_DTYPE_Q8_0 && d.down.dtype != VITNA_DTYPE_Q8_0);
+    const bool q8 = d.gate.dtype == VITNA_DTYPE_Q8_0 || d.down.dtype == VITNA_DTYPE_Q8_0;
+    if (rows_fast(g, n)) return !q8;
+    return n >= GSX_FEW_ROWS || q8 || gsx_least_blocks(d.gate, g->E) > GSX_FEW_BLOCKS;
 }
 
 /* A fast pass's working buffers for the layers that take the prefill's kernels, if any does. */

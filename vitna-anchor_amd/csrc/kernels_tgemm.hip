@@ -403,13 +403,15 @@ __device__ __forceinline__ int tg_item(int n) {
 bool gsx_fits(const qmat& gate, const qmat& up, const qmat& down) {
     auto dt = [](int d) { return d == VITNA_DTYPE_Q8_0 || d == VITNA_DTYPE_Q4_K || d == VITNA_DTYPE_Q6_K; };
     const int H = gate.cols, I = gate.rows;
-    /* whole superblocks, at most eight a row (one block's waves), whole 32-row tiles */
+    /* whole superblocks of the width and whole blocks of rows; experts wider than 2048 keep the four-pair kernels, as
+       none has been timed here */
     return dt(gate.dtype) && up.dtype == gate.dtype && dt(down.dtype) && up.rows == I && up.cols == H && down.rows == H &&
            down.cols == I && H % 256 == 0 && I % 256 == 0 && H <= 2048 && I <= 2048;
 }
 
 int gsx_max_tiles(int n, int K, int E) { return (n * K + 31) / 32 + E; }
 int gsx_max_blocks(int n, int K, int E) { return (n * K + 63) / 64 + E; }
+int gsx_least_blocks(const qmat& gate, int E) { return E * std::min(gate.rows / 128, gate.cols / 256); }
 
 __device__ __forceinline__ float gsx_largest(float m, const float4& v) {
     return fmaxf(m, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));

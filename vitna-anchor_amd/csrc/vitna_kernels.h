@@ -340,6 +340,8 @@ bool gsx_fits(const qmat& gate, const qmat& up, const qmat& down);
 int gsx_max_tiles(int n, int K, int E);
 /* The most token blocks of the grouped experts: two tiles (a fast pass: four) of one expert each. */
 int gsx_max_blocks(int n, int K, int E);
+/* The blocks of the smaller of its two kernels when every expert has one token block. */
+int gsx_least_blocks(const qmat& gate, int E);
 size_t gsx_tiled_bytes(const qmat& m, int n_experts);
 hipError_t launch_gsx_tile(const qmat& m, int n_experts, uint8_t* dst, hipStream_t s);
 hipError_t launch_gsx(const gsx_args& a, hipStream_t s);
