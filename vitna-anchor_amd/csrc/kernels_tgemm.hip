@@ -432,8 +432,12 @@ __global__ __launch_bounds__(256) void gsx_plan_kernel(const int* __restrict__ c
         const int row = 4 * (blockIdx.x - 1) + wv;
         if (row >= n) return;
         const float4* src = reinterpret_cast<const float4*>(x + (size_t)row * H);
+        float4 v[8]; /* gsx_fits: at most 2048 wide */
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] = 256 * i < H ? src[lane + 64 * i] : make_float4(0.f, 0.f, 0.f, 0.f);
         float m = 0.0f;
-        for (int c = lane; c < H / 4; c += 64) m = gsx_largest(m, src[c]);
+#pragma unroll
+        for (int i = 0; i < 8; i++) m = gsx_largest(m, v[i]);
 #pragma unroll
         for (int d = 1; d < 64; d <<= 1) m = fmaxf(m, __shfl_xor(m, d, WAVE));
         if (lane == 0) scale[row] = th_scale(m);
@@ -567,7 +571,7 @@ __device__ __forceinline__ void gsx_put(u32x4* img, bool order_b, bool fast, int
     img[((size_t)(row >> 5) * (K / 256) + (c8 >> 5)) * 1024 + (U * 4 + i) * 64 + (row & 31) + 32 * kq] = vh;
 }
 
-/* The images (one column order) and, for Q4_K weights, group sums of the virtual token tiles: block (b, t) takes
+/* The images (one column order) and, for Q4_K weights (sums not null), group sums of the virtual token tiles: block (b, t) takes
    superblock b of tile t, whose token l is pair 32 (t - toff[e]) + l of expert te[t] (past its count: the last pair
    again), row pair / ROUTE_K_MAX of x, times that row's scale, whose inverse goes to inv. */
 __global__ __launch_bounds__(256) void gsx_image_kernel(const float* __restrict__ x, int K, const float* __restrict__ scale,
@@ -587,12 +591,12 @@ __global__ __launch_bounds__(256) void gsx_image_kernel(const float* __restrict_
         const float4 v0 = src[0], v1 = src[1];
         const float ev[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
         const float f = scale[src_row];
-        if (c8 == 0) inv[32 * t + l] = 1.0f / f;
+        if (c8 == 0) inv[32 * t + l] = th_inverse(f);
         u32x4 vh, vl;
         float sum;
         th_split8(ev, f, fast, vh, vl, sum);
         gsx_put(img, order_b, fast, 32 * t + l, K, c8, vh, vl);
-        if (order_b) continue;
+        if (!sums) continue;
         const float t16 = sum + __shfl_xor(sum, 1, WAVE), t32 = t16 + __shfl_xor(t16, 2, WAVE);
         if (!(c8 & 3)) th_sum(sums + ((size_t)t * (K / 256) + b) * 1024, l, (c8 & 31) >> 2, t32);
     }
@@ -613,7 +617,7 @@ __global__ __launch_bounds__(256) void gsx_act_image_kernel(const float* __restr
 #pragma unroll
     for (int d = 1; d < 8; d <<= 1) m = fmaxf(m, __shfl_xor(m, d, WAVE));
     const float f = th_scale(m);
-    if (j == 0) inv[row] = 1.0f / f;
+    if (j == 0) inv[row] = th_inverse(f);
     for (int c = j; c < K / 8; c += 8) {
         const float4 v0 = src[2 * c], v1 = src[2 * c + 1];
         const float ev[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
@@ -621,7 +625,7 @@ __global__ __launch_bounds__(256) void gsx_act_image_kernel(const float* __restr
         float sum;
         th_split8(ev, f, fast, vh, vl, sum);
         gsx_put(img, order_b, fast, row, K, c, vh, vl);
-        if (order_b) continue;
+        if (!sums) continue;
         const float t16 = sum + __shfl_xor(sum, 1, WAVE), t32 = t16 + __shfl_xor(t16, 2, WAVE);
         if (!(c & 3)) th_sum(sums + ((size_t)t * (K / 256) + (c >> 5)) * 1024, l, (c & 31) >> 2, t32);
     }
@@ -661,9 +665,11 @@ hipError_t launch_gsx(const gsx_args& a, hipStream_t s) {
     u32x4* ia = reinterpret_cast<u32x4*>(a.img_act);
     _Float16* sums = reinterpret_cast<_Float16*>(a.sums);
     gsx_image_kernel<<<dim3(H / 256, T), 256, 0, s>>>(a.xn, H, a.scale, a.pairs, a.count, a.cap, a.toff, a.te, ii,
-                                                      a.gate.dtype == VITNA_DTYPE_Q6_K, a.fast, sums, a.inv);
+                                                      a.gate.dtype == VITNA_DTYPE_Q6_K, a.fast,
+                                                      a.gate.dtype == VITNA_DTYPE_Q4_K ? sums : nullptr, a.inv);
     hipError_t err = a.fast ? launch_gsx_tiles<true>(a, true, s) : launch_gsx_tiles<false>(a, true, s);
     if (err != hipSuccess) return err;
-    gsx_act_image_kernel<<<T, 256, 0, s>>>(a.act, I, a.te, ia, a.down.dtype == VITNA_DTYPE_Q6_K, a.fast, sums, a.inv);
+    gsx_act_image_kernel<<<T, 256, 0, s>>>(a.act, I, a.te, ia, a.down.dtype == VITNA_DTYPE_Q6_K, a.fast,
+                                       a.down.dtype == VITNA_DTYPE_Q4_K ? sums : nullptr, a.inv);
     return a.fast ? launch_gsx_tiles<true>(a, false, s) : launch_gsx_tiles<false>(a, false, s);
 }

@@ -53,6 +53,9 @@ __device__ __forceinline__ float th_scale(float largest) {
     return e == 0xff ? 1.0f : __uint_as_float((uint32_t)(min(13 - (e - 127), 126) + 127) << 23);
 }
 
+/* 1 / f of a power of two whose inverse is normal */
+__device__ __forceinline__ float th_inverse(float f) { return __uint_as_float((254u << 23) - __float_as_uint(f)); }
+
 /* eight values times f as f16 hi and lo in the operands' order, and the sum of hi + lo (fast: of hi) */
 __device__ __forceinline__ void th_split8(const float e[8], float f, bool fast, u32x4& vh, u32x4& vl, float& sum) {
     h8 h, l;
