@@ -432,12 +432,8 @@ __global__ __launch_bounds__(256) void gsx_plan_kernel(const int* __restrict__ c
         const int row = 4 * (blockIdx.x - 1) + wv;
         if (row >= n) return;
         const float4* src = reinterpret_cast<const float4*>(x + (size_t)row * H);
-        float4 v[8]; /* gsx_fits: at most 2048 wide */
-#pragma unroll
-        for (int i = 0; i < 8; i++) v[i] = 256 * i < H ? src[lane + 64 * i] : make_float4(0.f, 0.f, 0.f, 0.f);
         float m = 0.0f;
-#pragma unroll
-        for (int i = 0; i < 8; i++) m = gsx_largest(m, v[i]);
+        for (int c = lane; c < H / 4; c += 64) m = gsx_largest(m, src[c]);
 #pragma unroll
         for (int d = 1; d < 64; d <<= 1) m = fmaxf(m, __shfl_xor(m, d, WAVE));
         if (lane == 0) scale[row] = th_scale(m);
