@@ -547,8 +547,8 @@ hipError_t launch_attention(const attn_args& a, hipStream_t s) {
    RW = 16 / G rows of the tile times the G heads, against the chunk's 64 positions, each row masked to the
    positions up to its own. The queries come prepared (launch_attention_prepare). The scores of each chunk fold
    into a running maximum and sum per column, the values into O rescaled as the maximum grows, and the block
-   writes att itself (O / sum): no chunk leaves a partial and no merge runs. Passes of more than 64 rows reach it (the exact-rows limit), so it is held to 1e-3, not to a step's
-   bits.
+   writes att itself (O / sum): no chunk leaves a partial and no merge runs. Passes of more than 64 rows reach it (the
+   exact-rows limit), so it is held to 1e-3, not to a step's bits.
 
    The products run on the bf16 matrix cores. Each operand is split into bf16 hi + lo (lo the rounding of what hi
    leaves) and each product taken as hi*hi + hi*lo + lo*hi on v_mfma_f32_16x16x32_bf16, summed in fp32: about
@@ -814,18 +814,22 @@ __global__ __launch_bounds__(256, 2) void attention_flash_kernel(attn_args a) {
     }
 }
 
-/* Row tiles from which the chunks' images pay. 42 tiles of 333 rows from position 0 (at most 6 chunks) took 33.1 us
-   splitting their own and 26.5 + 5.4 with images, and the more chunks, the more there is to repeat; below eight tiles a
-   launch is a larger share than what is repeated. */
+/* Row tiles and chunks from which the chunks' images pay: with few tiles they are read by few, with few chunks there is
+   little to repeat beside the launch. The grid's chunks are a power of two or all the cache has, so five means more than
+   four. Rows steps of four layers (32 query, 4 kv heads), without images and with, us: 65 rows (nine tiles) from
+   position 0 886 and 900, from 64 890 and 900, from 256 941 and 934, from 1024 1171 and 1083; 256 rows from 0 1229 and
+   1240, from 256 1221 and 1210; 333 rows from 0 level; 512 from 0 1721 and 1713; 1024 2678 and 2636. */
 #define FL_IMAGE_TILES 8
+#define FL_IMAGE_CHUNKS 5
 
 hipError_t launch_attention_flash(const attn_args& a, hipStream_t s) {
     if (!attention_run_fits(a) || a.n_rows < 1) return hipErrorInvalidValue;
     const int G = a.n_heads / a.n_kv, tq = 4 * (16 / G);
     const dim3 grid(a.n_kv, (a.n_rows + tq - 1) / tq);
     /* (a.partial holds n_rows x n_heads x splits_max x (hd + 4) floats or more: a chunk's image takes 128 rows of one head) */
-    const bool imaged = (int)grid.y >= FL_IMAGE_TILES && (size_t)a.partial_rows * a.n_heads * (a.hd + 4) >= (size_t)a.n_kv * FL_IMAGE;
-    if (imaged) attention_image_kernel<<<dim3(a.n_kv, a.splits_grid > 0 ? a.splits_grid : a.splits_max), 256, 0, s>>>(a);
+    const int chunks = a.splits_grid > 0 ? a.splits_grid : a.splits_max;
+    const bool imaged = (int)grid.y >= FL_IMAGE_TILES && chunks >= FL_IMAGE_CHUNKS && (size_t)a.partial_rows * a.n_heads * (a.hd + 4) >= (size_t)a.n_kv * FL_IMAGE;
+    if (imaged) attention_image_kernel<<<dim3(a.n_kv, chunks), 256, 0, s>>>(a);
     switch (imaged ? G : -G) {
         case 8: attention_flash_kernel<8, true><<<grid, 256, 0, s>>>(a); break;
         case 4: attention_flash_kernel<4, true><<<grid, 256, 0, s>>>(a); break;
