@@ -689,8 +689,8 @@ extern "C" struct vitna_cuda_model* vitna_cuda_create(const vitna_llama_t* m, co
         return bail();
     }
     g->seq_seen.resize(m->seqs);
-    g->results = host_copy_create();
-    if (!g->results || hipHostMalloc((void**)&g->rows_host, R * sizeof(row_rec), 0) != hipSuccess ||
+    g->results = host_copy_create(); /* without it results are copied a row at a time */
+    if (hipHostMalloc((void**)&g->rows_host, R * sizeof(row_rec), 0) != hipSuccess ||
         hipHostMalloc((void**)&g->h_logits, 2 * R * E * 4, 0) != hipSuccess ||
         hipHostMalloc((void**)&g->rt_host, R * sizeof(route_out), 0) != hipSuccess) {
         fail(err, err_len, "page-locked host memory for the rows and logits");
