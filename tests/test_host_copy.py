@@ -1,8 +1,8 @@
 """The results' way to the host (csrc/host_copy.hip) on the CPU: its source compiled against a stand-in for the HIP runtime
 whose copies are queued and done when something waits for them, so that bytes taken before they arrived are wrong ones.
 
-Every row's bytes, rows that were not asked for untouched, memory that HIP allocated (page-locked, device) written by the
-device itself, and a model without page-locked chunks still served.
+Every row's bytes, rows that were not asked for untouched, rows with gaps waited for together, memory that HIP allocated
+(page-locked, device) written by the device itself, and a model without page-locked chunks still served.
 """
 import ctypes as C
 import os
@@ -146,6 +146,18 @@ def test_bytes(copier, n, bytes_):
     for want in (range(n), [0], [n - 1], range(0, n, 2), range(n // 3, n), []):
         for stride in (None, bytes_ + 64):
             assert Rows(n, bytes_, want, stride).run(lib, c)[0] == 0
+
+
+def test_gaps_are_waited_for_once(lib):
+    """Small rows with gaps: one wait, nothing copied past the chunks; more runs than are held, or than 16 MB hold, a wait
+    for each lot."""
+    c = lib.make(0)
+    assert Rows(200, 4000, range(0, 200, 2)).run(lib, c) == (0, 1, 0)
+    assert Rows(64, 4000, [0, 1, 5, 6, 7, 60]).run(lib, c) == (0, 1, 0)
+    assert Rows(1024, 400, range(0, 1024, 2)).run(lib, c) == (0, 1, 0)
+    assert Rows(2048, 400, range(0, 2048, 2)).run(lib, c) == (0, 2, 0)
+    assert Rows(1024, 65536, range(0, 1024, 2)).run(lib, c) == (0, 2, 0)
+    lib.unmake(c)
 
 
 def test_memory_of_hip_is_written_directly(lib):
