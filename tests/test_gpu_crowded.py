@@ -1,6 +1,7 @@
 """Crowded passes: a pass of many rows puts tens of pairs on every expert (a prompt's chunk of 1024 rows of top-8
-over 128 experts: 64 an expert). From 512 rows on, a model whose experts are resident runs them on tiles of 32
-pairs of one expert (launch_gsx in kernels_skinny.hip) instead of the four-pair tiles of kernels_gmma.hip.
+over 128 experts: 64 an expert). From 64 rows on (96 for small K-quant experts), a model whose experts are resident
+runs them on tiles of 32 pairs of one expert (launch_gsx in kernels_tgemm.hip) instead of the four-pair tiles of
+kernels_gmma.hip.
 
 The bar is the grouped kernels': each layer, the device's residual rows before and after
 vitna_cuda_moe_rows_experts (routed by the host from the device's router logits, as model.c routes a prompt's

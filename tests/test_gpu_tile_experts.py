@@ -215,3 +215,30 @@ def test_first_tiled_passes(experts, gate_up, down, n):
     finally:
         dev.close()
         model.free()
+
+
+@pytest.mark.parametrize("gate_up,down,fast", [(a, b, f) for a, b in ((va.Q4_K, va.Q4_K), (va.Q6_K, va.Q6_K), (va.Q4_K, va.Q6_K))
+                                               for f in (False, True)] + [(va.Q8_0, va.Q8_0, False)])
+def test_widest_experts(gate_up, down, fast):
+    """Experts of 2048 x 2048, the widest on the tiles (a fast pass's Q8_0 ones keep the prefill's kernel): some of 97 rows,
+    two experts each, to the bars above."""
+    say("widest experts", gate_up, down, fast)
+    n, E, K = 97, 8, 2
+    model = va.Model(va.shape(n_layers=1, hidden=2048, intermediate=2048, n_heads=4, n_kv_heads=2, head_dim=64, vocab=300, n_experts=E,
+                              n_experts_used=K, renormalize=0, dt_gate_up=gate_up, dt_down=down, norm_std=0.5, ctx=n, seqs=1), 982)
+    dev = va.Device(model, fast=fast)
+    try:
+        x0, xn = given_rows(model, dev, n)
+        rng = np.random.RandomState(4)
+        ids = np.stack([np.sort(rng.choice(E - 1, K, replace=False)) for _ in range(n)]).astype(np.int32)
+        w = rng.uniform(0.05, 1.0, (n, K)).astype(np.float32)
+        dev.rows_experts(0, ids, w)
+        for i in range(0, n, 12):
+            ref, bound = fast_bound(model, 0, xn[i], ids[i], w[i])
+            got = dev.residual(i).astype(np.float64) - x0[i]
+            most = float(np.max(np.abs(ref)))
+            lost = float(np.max(np.abs(x0[i] + ref))) * 2.0 ** -23
+            assert np.max(np.abs(got - ref) / (bound + lost) if fast else np.abs(got - ref) / (REL * most + lost)) <= 1.0, ("row", i)
+    finally:
+        dev.close()
+        model.free()

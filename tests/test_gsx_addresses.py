@@ -193,6 +193,9 @@ def check(n, K, E, H, I, ids, fast, gate_up="Q4_K", down="Q6_K"):
                             for src, at, lds, size in loads(dt, fast, S, tt, wv, b, U, part):
                                 limit = {"img": have[img], "sums": have["sums"], "wt": S * L.TB}[src]
                                 assert 0 <= at and at + size <= limit, (src, at)
+                                if src != "wt":  # this superblock of one of the block's tiles
+                                    per = 2048 if src == "sums" else 16384 if fast else 32768
+                                    assert at // (S * per) in tt and at // per % S == b and (at + size - 1) // per == at // per
                                 assert lds % 16 == 0 and lds + size <= L.BYTES
         assert L.BYTES <= 160 * 1024
     # the results: gate/up's rows of the tiles that there are, down's pairs
