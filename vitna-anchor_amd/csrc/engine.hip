@@ -129,7 +129,9 @@ struct vitna_cuda_model {
     uint32_t *gsx_img_in, *gsx_img_act;
     uint16_t* gsx_sums;
     float *gsx_act, *gsx_scale, *gsx_inv;
-    std::vector<uint64_t> seq_seen; /* by sequence: the last pass (seq_pass) that had a row of it */
+    /* the sequences of the pass seq_pass, each in the first free slot from its number on; twice a pass's rows, whatever
+       the model's seqs */
+    struct { uint64_t pass; int seq; } seq_seen[2 * ROWS_MAX];
     uint64_t seq_pass;
     bool rows_shared_seq;       /* the pass's rows include two of one sequence (attention prepares first) */
     bool rows_one_seq;          /* every row of the pass is of one sequence (a prompt's chunk: tiles of rows) */
@@ -688,7 +690,6 @@ extern "C" struct vitna_cuda_model* vitna_cuda_create(const vitna_llama_t* m, co
         fail(err, err_len, "clearing device scratch failed");
         return bail();
     }
-    g->seq_seen.resize(m->seqs);
     g->results = host_copy_create(); /* without it results are copied a row at a time */
     if (hipHostMalloc((void**)&g->rows_host, R * sizeof(row_rec), 0) != hipSuccess ||
         hipHostMalloc((void**)&g->h_logits, 2 * R * E * 4, 0) != hipSuccess ||
@@ -2380,8 +2381,10 @@ static bool set_rows(vitna_cuda_model* g, const vitna_cuda_row_t* rows, size_t n
         if (r.seq < 0 || r.seq >= g->seqs) return fail(err, err_len, "row %zu: sequence %d, the cache holds %d", i, r.seq, g->seqs);
         if (r.pos < 0 || r.pos >= g->ctx) return fail(err, err_len, "row %zu: position %d, the cache holds %d", i, r.pos, g->ctx);
         if (r.token < 0 || r.token >= g->V) return fail(err, err_len, "row %zu: token %d outside the vocabulary of %d", i, r.token, g->V);
-        shared |= g->seq_seen[r.seq] == pass;
-        g->seq_seen[r.seq] = pass;
+        int at = r.seq % (2 * ROWS_MAX);
+        while (g->seq_seen[at].pass == pass && g->seq_seen[at].seq != r.seq) at = (at + 1) % (2 * ROWS_MAX);
+        shared |= g->seq_seen[at].pass == pass;
+        g->seq_seen[at] = {pass, r.seq};
     }
     HIP_TRY(hipEventSynchronize(g->rows_copied), "waiting for the previous row copy");
     g->row_set = false;
