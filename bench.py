@@ -320,8 +320,8 @@ def bench_prompt(va, model, tokens=4096, chunk=1024):
     rows of one sequence at consecutive positions, in a cache of `tokens` positions (model.c's default context is the
     model's, at most 4096), as model.c feeds a prompt in chunks of vitna_cuda_moe_rows_max
     (the rows step: each row's attention over the keys of the positions before it and its own, device routing,
-    experts grouped), with the exact kernels and with --precision fast (a gpu_fast model: the passes' experts as
-    the bf16 grouped GEMM). The last position's logits come back, as model.c asks of a prompt. Wall-clock of the
+    experts grouped), with the exact kernels and with --precision fast (a gpu_fast model: the passes' experts in
+    16-bit activations). The last position's logits come back, as model.c asks of a prompt. Wall-clock of the
     second prompt (the first captures the graphs and makes the tiled copies)."""
     cfg = model.cfg
     out = {"workload": "a %d-token prompt through BASELINE configs[2]'s model (Qwen3-30B-A3B-shaped Q4_K_M, 48 layers), "

@@ -2252,7 +2252,7 @@ static hipError_t enqueue_rows_head(vitna_cuda_model* g, int n, const float* ypa
                                         img ? model_img(g) : img_out{nullptr, nullptr, nullptr, nullptr}, g->stream);
     if (e != hipSuccess || head == HEAD_NONE) return e;
     if (head >= 0) {
-        /* one row: the decode step's GEMV (151936 x 2048 Q6_K 105 us on the multi-row GEMV, 47 on it) */
+        /* one row: the decode step's GEMV (151936 x 2048 Q6_K 105 us on the multi-row GEMV, 57 on it) */
         gemv_args a;
         memset(&a, 0, sizeof(a));
         a.w[0] = g->head; a.n = 1; a.norm_w = g->final_norm; a.eps = g->eps;

@@ -26,15 +26,17 @@
  * of among them, the stage took 2200 clocks. A wave with one superblock of one
  * tile and its sums added through LDS (the kernels before) waited for its
  * first loads most of its life. One layer's experts of a 1024-row pass (top-8
- * of 128, 2048 x 768; kernel trace): gate/up in Q4_K 293 -> 163 us, down in
- * Q6_K 243 -> 173 us; 333 rows in Q8_0 155 -> 112 and 113 -> 74 us.
+ * of 128, 2048 x 768; kernel trace): gate/up in Q4_K 293 -> 167 us (163 with
+ * group sums of 22 bits), down in Q6_K 243 -> 173 us; 333 rows in Q8_0 155 ->
+ * 95 to 135 by how the rows fall on the experts, and 113 -> 80 us.
  *
  * A --precision fast pass takes the activations' hi alone: a wave's second
  * token tile takes the place of the first one's lo, so a block holds four
  * tiles of one expert and each weight is unpacked for two. Against the bf16
  * GEMM that widened each K-quant weight in float32 (kernels_prefill.hip): 246
- * -> 131 and 181 -> 135 us at the same sizes, the error against 64 bits of a
- * two-layer pass 6e-3 -> 4e-4 (f16 keeps 11 bits, bf16 8).
+ * -> 139 and 181 -> 138 us at the same sizes (135 with the first piece of the
+ * group sums alone), the error against 64 bits of a two-layer pass 6e-3 -> 5e-4
+ * (f16 keeps 11 bits, bf16 8).
  */
 
 #include "vitna_kernels.h"
